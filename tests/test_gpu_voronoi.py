@@ -117,3 +117,68 @@ def test_model_refresh_warm_start(gpu):
     adj, off, _ = ops.build_voronoi_adjacency(m.primal_points)
     torch.cuda.synchronize()
     assert torch.equal(m.point_adjacency, adj) and torch.equal(m.point_adjacency_offsets, off)
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 7, 8, 9, 63, 64, 65, 66, 511, 512, 513, 32767, 32769, 65535, 65537])
+def test_site_counts_at_tree_edges(gpu, n):
+    """Site counts around the builder's groups (8 sites per leaf box, 64 boxes
+    per box above, 64 seeds per cell) and around the count from which its
+    sort takes all Morton bits.  Up to 4 sites in general position are all
+    neighbours of each other."""
+    pts = np.random.default_rng(100 + n).uniform(-1, 1, size=(n, 3)).astype(np.float32)
+    if n >= 5:
+        _check(pts, gpu)
+        return
+    adj, off, _ = ops.build_voronoi_adjacency(H.to_dev(pts, gpu))
+    adj, off = adj.cpu().numpy(), off.cpu().numpy()
+    for i in range(n):
+        assert np.array_equal(adj[off[i]:off[i + 1]], [j for j in range(n) if j != i])
+
+
+@pytest.mark.parametrize("faces", [30, 40, 64, 65, 120, 230])
+def test_cell_with_many_faces(gpu, faces):
+    """A site inside a sphere of others has them all as neighbours: cells of one
+    vertex per lane, of two and of eight, and lists longer than a slot."""
+    d = np.random.default_rng(faces).normal(size=(faces, 3))
+    shell = d / np.linalg.norm(d, axis=1, keepdims=True) * np.array([1.0, 0.97, 0.94])
+    pts = np.concatenate([[[0.01, -0.02, 0.015]], shell]).astype(np.float32)
+    _check(pts, gpu)
+
+
+@pytest.mark.parametrize("scale", [1e-6, 1.0, 1e6])
+def test_clusters_of_very_different_density(gpu, scale):
+    """Clusters a thousandth of the scene wide beside sparse sites (a Morton
+    grid coarser than a cluster, reaches that differ a thousandfold)."""
+    rng = np.random.default_rng(8)
+    sparse = rng.uniform(-1, 1, size=(3000, 3))
+    dense = [c + 1e-3 * rng.normal(size=(700, 3)) for c in rng.uniform(-1, 1, size=(3, 3))]
+    _check((scale * np.concatenate([sparse, *dense])).astype(np.float32), gpu)
+
+
+def test_sites_on_common_spheres(gpu):
+    """Sites on a 1/64 grid (no two alike): many fives on common spheres, whose
+    Delaunay neighbours are not unique.  The build succeeds and gives the
+    neighbours that share a face of some area: those that qhull finds however
+    the sites are moved by less than matters."""
+    pts = np.unique(np.round(np.random.default_rng(0).uniform(-1, 1, size=(3000, 3)) * 64) / 64, axis=0)
+    adj, off, _ = ops.build_voronoi_adjacency(H.to_dev(pts.astype(np.float32), gpu))
+    adj, off = adj.cpu().numpy().astype(np.int64), off.cpu().numpy().astype(np.int64)
+    n = pts.shape[0]
+
+    def pairs(a, o):
+        return set(zip(np.repeat(np.arange(n), np.diff(o.astype(np.int64))).tolist(), a[:o[-1]].tolist()))
+
+    sure = None
+    for seed in range(24):
+        got = pairs(*scene.delaunay_csr(pts + 1e-9 * np.random.default_rng(seed).normal(size=pts.shape), pad=0))
+        sure = got if sure is None else sure & got
+    assert pairs(adj, off) == sure
+
+
+def test_lattice(gpu):
+    """A cubic lattice: the neighbours along the axes, none across edges or corners."""
+    g = np.stack(np.meshgrid(*[np.arange(10)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    adj, off, _ = ops.build_voronoi_adjacency(H.to_dev(g.astype(np.float32), gpu))
+    adj, off = adj.cpu().numpy(), off.cpu().numpy()
+    for i in range(len(g)):
+        assert np.array_equal(adj[off[i]:off[i + 1]], np.flatnonzero(np.abs(g - g[i]).sum(1) == 1))

@@ -256,8 +256,13 @@ __global__ void bbox_init_kernel(int32_t *ws)
         ws[threadIdx.x] = (int32_t)0x80000000;
 }
 
-__global__ __launch_bounds__(256) void bbox_reduce_kernel(const float *__restrict__ p, uint32_t n, int32_t *ws)
+// The blocks meet in 6 words by atomics, about 12 ns each on one address: few
+// large blocks with one set of atomics each (1M points: 282 us with 1,024
+// blocks of 4 waves, an atomic per wave).
+constexpr uint32_t BBOX_THREADS = 1024, BBOX_BLOCKS = 128;
+__global__ __launch_bounds__(BBOX_THREADS) void bbox_reduce_kernel(const float *__restrict__ p, uint32_t n, int32_t *ws)
 {
+    __shared__ int32_t part[6][BBOX_THREADS / 64];
     int32_t lo[3] = {0x7fffffff, 0x7fffffff, 0x7fffffff};
     int32_t hi[3] = {(int32_t)0x80000000, (int32_t)0x80000000, (int32_t)0x80000000};
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
@@ -279,9 +284,19 @@ __global__ __launch_bounds__(256) void bbox_reduce_kernel(const float *__restric
     if ((threadIdx.x & 63) == 0) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            atomicMin(ws + c, lo[c]);
-            atomicMax(ws + 3 + c, hi[c]);
+            part[c][threadIdx.x >> 6] = lo[c];
+            part[3 + c][threadIdx.x >> 6] = hi[c];
         }
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        int32_t v = part[threadIdx.x][0];
+        for (uint32_t w = 1; w < BBOX_THREADS / 64; ++w)
+            v = threadIdx.x < 3 ? min(v, part[threadIdx.x][w]) : max(v, part[threadIdx.x][w]);
+        if (threadIdx.x < 3)
+            atomicMin(ws + threadIdx.x, v);
+        else
+            atomicMax(ws + threadIdx.x, v);
     }
 }
 
@@ -296,8 +311,8 @@ int bbox3(const float *points, uint32_t n, float *bbox6, uint32_t *ws, hipStream
     bbox_init_kernel<<<1, 64, 0, s>>>((int32_t *)ws);
     VT_LAUNCH_CHECK("bbox_init_kernel");
     if (n > 0) {
-        uint32_t blocks = min((n + 255u) / 256u, 1024u);
-        bbox_reduce_kernel<<<blocks, 256, 0, s>>>(points, n, (int32_t *)ws);
+        uint32_t blocks = min((n + BBOX_THREADS - 1) / BBOX_THREADS, BBOX_BLOCKS);
+        bbox_reduce_kernel<<<blocks, BBOX_THREADS, 0, s>>>(points, n, (int32_t *)ws);
         VT_LAUNCH_CHECK("bbox_reduce_kernel");
     }
     bbox_final_kernel<<<1, 64, 0, s>>>((const int32_t *)ws, bbox6);
