@@ -1,0 +1,123 @@
+"""Launches of few tiles run with four lanes per ray, larger ones with one
+(vt_walk.h walk_step_group, the *_GROUP_TILES rules): the same rays rendered or
+trained in a small launch and inside a large one give the same bits per ray,
+and the same gradients up to the order of their sums.  The small launches are
+held against the oracle by the other tests' frames."""
+import numpy as np
+import pytest
+import torch
+
+from tests import helpers as H
+from vorotracing_amd import _C, camera, scene
+from vorotracing_amd.infer import VoroTracingInfer
+from vorotracing_amd.model import VoroTracing
+
+pytestmark = pytest.mark.gpu
+
+MOST = 3072  # tiles of the largest launch with four lanes per ray
+
+
+def _images(gpu, n, h, w):
+    """n images of one camera each (n, h, w, 6)."""
+    return H.to_dev(np.stack([camera.orbit_rays(k, w, h, n=n, radius=4.0) for k in range(n)]), gpu)
+
+
+def _tiles(rays):
+    if rays.dim() == 2:
+        return (rays.shape[0] + 63) // 64
+    b = 1 if rays.dim() == 3 else rays.shape[0]
+    return b * ((rays.shape[-3] + 7) // 8) * ((rays.shape[-2] + 7) // 8)
+
+
+@pytest.mark.parametrize("h,w", [(121, 131), (8, 9), (64, 64)])
+@pytest.mark.parametrize("quantize", ["fp16", "q8"])
+def test_render_small_and_large_launch(gpu, quantize, h, w):
+    m = VoroTracing.from_scene(scene.random_scene(1500, seed=3, R=8, Rs=4), device=gpu)
+    inf = VoroTracingInfer(m, quantize=quantize)
+    n = MOST // _tiles(_images(gpu, 1, h, w)[0]) + 1
+    rays = _images(gpu, n, h, w)
+    assert _tiles(rays) > MOST >= _tiles(rays[0])
+    kw = dict(weight_threshold=0.001, cell_skip_threshold=1e-3)
+    whole = inf.render(rays, **kw)
+    for k in (0, n // 2, n - 1):
+        assert torch.equal(inf.render(rays[k].contiguous(), **kw), whole[k])
+    flat = rays[:, ::3, ::2].reshape(-1, 6).contiguous()
+    flat = flat.repeat(-(-(64 * MOST + 1) // flat.shape[0]), 1)
+    start = inf.bvh.start_cells(inf.primal_points, flat)
+    whole = inf.render(flat, start_point=start, **kw)
+    for count in (1, 63, 65, 1001):
+        assert torch.equal(inf.render(flat[:count].contiguous(), start_point=start[:count].contiguous(), **kw),
+                           whole[:count])
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("h,w", [(121, 131), (9, 8)])
+def test_training_small_and_large_launch(gpu, f16, h, w):
+    """Every per-ray output of the forward bit for bit (depth quantiles and
+    statistics of the distortion among them); contribution and gradients of the
+    large launch against the sums over the small ones."""
+    s = scene.random_scene(1200, seed=5, R=4, Rs=8)
+    m = VoroTracing.from_scene(s, device=gpu)
+    dt = torch.float16 if f16 else torch.float32
+    scn = (m.primal_points.detach(), m.att_diffuse.detach().to(dt), m.att_specular.detach().to(dt),
+           m.activated_density().detach(), m.point_adjacency, m.point_adjacency_offsets)
+    n = MOST // _tiles(_images(gpu, 1, h, w)[0]) + 1
+    rays = _images(gpu, n, h, w)
+    assert _tiles(rays) > MOST
+    g = torch.Generator(device=gpu).manual_seed(1)
+    start = m.get_starting_point(rays)
+    lead = list(rays.shape[:-1])
+    q = torch.tensor([0.7, 0.3], device=gpu).expand(lead + [2]).contiguous()
+    # upstream gradients for a few of the images: the others add nothing
+    some = sorted({0, n // 2, n - 1})
+    up = torch.zeros(lead + [4], device=gpu)
+    gd = torch.zeros(lead + [1], device=gpu)
+    gq = torch.zeros(lead + [2], device=gpu)
+    for k in some:
+        up[k] = torch.randn(up[k].shape, generator=g, device=gpu)
+        gd[k] = 0.01 * torch.rand(gd[k].shape, generator=g, device=gpu)
+        gq[k] = 0.1 * torch.randn(gq[k].shape, generator=g, device=gpu)
+    up = up.to(dt)
+
+    def both(sel):
+        r, sp, qs = rays[sel].contiguous(), start[sel].contiguous(), q[sel].contiguous()
+        out = _C.trace_vorotracing_fwd(*scn, r, sp, qs, 0.001, 1024, True)
+        rgba, depth, idx, _, _, dist, wt, st, tf = out
+        err = torch.ones(list(r.shape[:-1]) + [1], dtype=dt, device=gpu) * 0.5
+        grads = _C.trace_vorotracing_bwd(*scn, r, sp, rgba, up[sel].contiguous(), qs, idx, gq[sel].contiguous(), err, 0.0,
+                                         dist, gd[sel].contiguous(), wt, st, tf, 0.001, 1024)
+        return out, grads
+
+    whole, wgrads = both(slice(None))
+    parts = {k: both(k) for k in some}
+    for k, (out, _) in parts.items():
+        for name, a, b in zip(("rgba", "depth", "depth_idx", None, "n", "distortion", "W", "S", "t_far"), out, whole):
+            if name:
+                assert torch.equal(a.view(torch.int16 if a.dtype == torch.float16 else torch.int32),
+                                   b[k].view(torch.int16 if a.dtype == torch.float16 else torch.int32)), (k, name)
+    # sums in two orders: f32 atomics within 1e-5 of the tensor's norm, half ones (rounded at every add) within 2e-2
+    for i, tol in ((0, 1e-5), (1, 2e-2 if f16 else 1e-5), (2, 2e-2 if f16 else 1e-5), (3, 1e-5)):
+        want = wgrads[i].double()
+        got = sum(p[1][i].double() for p in parts.values())
+        assert float((got - want).norm()) <= tol * float(want.norm()), i
+
+
+def test_contribution_and_point_error(gpu):
+    """The lane that adds to the shared outputs adds once per ray: against a large launch of the same rays repeated."""
+    m = VoroTracing.from_scene(scene.random_scene(600, seed=9, R=4), device=gpu)
+    scn = (m.primal_points.detach(), m.att_diffuse.detach(), m.att_specular.detach(),
+           m.activated_density().detach(), m.point_adjacency, m.point_adjacency_offsets)
+    ray = _images(gpu, 1, 64, 72)
+    times = MOST // _tiles(ray[0]) + 1
+    sums = []
+    for rays in (ray[0], ray.repeat(times, 1, 1, 1)):
+        rays = rays.contiguous()
+        start = m.get_starting_point(rays)
+        out = _C.trace_vorotracing_fwd(*scn, rays, start, None, 0.001, 1024, True)
+        err = torch.ones(list(rays.shape[:-1]) + [1], device=gpu)
+        grads = _C.trace_vorotracing_bwd(*scn, rays, start, out[0], torch.zeros_like(out[0]), None, None, None, err, 0.0,
+                                         out[5], None, out[6], out[7], out[8], 0.001, 1024)
+        sums.append((out[3].double(), grads[5].double()))
+    for a, b in zip(sums[0], sums[1]):
+        assert float((times * a - b).norm()) <= 1e-5 * float(b.norm())
+        assert float(a.sum()) > 0

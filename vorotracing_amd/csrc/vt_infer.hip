@@ -151,14 +151,18 @@ struct ShadeQueue {
     float sw[4][64];                 // specular weights (tap-major: lanes of different owners on different banks)
     uint32_t tail;                   // entries appended so far (mod 2^32)
 };
-__shared__ ShadeQueue infer_queues[INFER_BLOCK / 64];
-
-__device__ __forceinline__ ShadeQueue &wave_queue() { return infer_queues[threadIdx.x >> 6]; }
+// (of the waves of the kernel's block)
+template <int WAVES> __device__ __forceinline__ ShadeQueue &wave_queue()
+{
+    __shared__ ShadeQueue infer_queues[WAVES];
+    return infer_queues[threadIdx.x >> 6];
+}
 
 // RayIntegratorOctMapInfer / ...InferQ8 (ray_integrator_octmap.cuh:315-344,
 // :487-515, colour :437-460).  A cell to shade goes to the wave's queue as
 // (cell, weight, probe offset); shade_batch computes its colour.
-template <int RD, int RS, class Tex> struct InferIntegrator {
+// G: lanes per ray, of which the first queues the cell and keeps the colour.
+template <int RD, int RS, class Tex, int G = 1> struct InferIntegrator {
     using TexType = Tex;
     f3 o, d;
     const float *density;
@@ -181,13 +185,13 @@ template <int RD, int RS, class Tex> struct InferIntegrator {
         float dt = __builtin_fmaxf(t1 - t0, 0.0f);
         float alpha = 1.0f - vt_expf(-s * dt);
         float w = T * alpha;
-        if (w >= skip) {
+        if (w >= skip && (G == 1 || threadIdx.x % G == 0)) {
             st.shade();
             // probe_dir's test len > 1e-8 on the squared length (exact, see PROBE_LEN2_MIN)
             const f3 dv = sub(mk(fma_(t0, d.x, o.x), fma_(t0, d.y, o.y), fma_(t0, d.z, o.z)), p);
             const bool tiny = !(dot(dv, dv) > PROBE_LEN2_MIN);
             // the lanes appending now are exactly the active ones
-            ShadeQueue &q = wave_queue();
+            ShadeQueue &q = wave_queue<G>();
             const uint64_t m = __ballot(1);
             const uint32_t rank = lane_rank(m), tail = q.tail;
             const uint32_t k = (tail + rank) & (SQ_RING - 1);
@@ -367,22 +371,10 @@ __device__ __forceinline__ uint32_t slot_to_ray(const InferArgs &a, uint32_t s, 
 }
 
 
-template <int RD, int RS, bool Q8, bool STATS, int MAP, int CHUNK, bool PACKED, bool QUADS>
-// 8 waves per SIMD need at most 64 VGPRs.  The fp16 kernel fits them; the q8
-// kernel spills 12 bytes per lane and is still faster than at 7 waves
-// (C4: 16.6 against 17.2 ms).  The statistics variants (tests and counters
-// only) keep their larger register budget.
-__global__ __launch_bounds__(INFER_BLOCK) __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 8)))
-void infer_kernel(InferArgs a, uint32_t total_slots)
+// The integrator of a launch, before its ray.
+template <bool Q8, bool QUADS, class Integ>
+__device__ __forceinline__ void begin_integrator(Integ &integ, const InferArgs &a)
 {
-    ShadeQueue &q = wave_queue();
-    const int lane = (int)(threadIdx.x & 63u);
-    // every lane stays in the wave's loop to the end (it shades for others)
-    const uint32_t s = xcd_interleaved_block<INFER_XCD_CHUNK>() * blockDim.x + threadIdx.x;
-    const uint32_t r = s < total_slots ? slot_to_ray(a, s, MAP) : NONE;
-    bool active = r != NONE;
-    using Tex = typename std::conditional<Q8, TexQ8<RD, RS, QUADS>, TexF16<RD, RS, QUADS>>::type;
-    InferIntegrator<RD, RS, Tex> integ;
     integ.density = a.density;
     if constexpr (Q8) {
         integ.tex.diffuse = (const uint8_t *)(QUADS ? a.quad_d : a.diffuse);
@@ -402,36 +394,74 @@ void infer_kernel(InferArgs a, uint32_t total_slots)
     integ.skip = a.skip;
     integ.acc = mk(0.0f, 0.0f, 0.0f);
     integ.T = 1.0f;
+}
+
+// Ray r of the launch and its specular taps (into the wave's queue); returns
+// its start cell.
+template <int RS, bool QUADS>
+__device__ __forceinline__ uint32_t begin_ray(const InferArgs &a, uint32_t r, bool camera, ShadeQueue &q, int lane, f3 &o,
+                                              f3 &d)
+{
+    uint32_t start;
+    if (camera) {
+        // the ray of pixel (u, v) of image img, normalised as load_ray does
+        const uint32_t hw = a.H * a.W, img = r / hw, rem = r - img * hw, v = rem / a.W, u = rem - v * a.W;
+        f3 dd;
+        camera_ray(a.cams[img], u, v, a.H, o, dd);
+        d = divs(dd, __builtin_sqrtf(dot(dd, dd)));
+        start = a.start_point[a.start_rows ? img * a.H + v : img];
+    } else {
+        load_ray(a.rays, r, o, d);
+        start = a.start_point[a.rays_per_start ? r / a.rays_per_start : r];
+    }
+    float su, sv;
+    oct_encode<RS>(mk(-d.x, -d.y, -d.z), su, sv);
+    Bilinear sb;
+    if constexpr (QUADS) {
+        sb = bilinear_quad<RS>(su, sv);
+        q.si[lane] = (uint32_t)sb.i00;
+    } else {
+        sb = bilinear_setup<RS>(su, sv);
+        q.si[lane] = (uint32_t)sb.i00 | (uint32_t)sb.i10 << 8 | (uint32_t)sb.i01 << 16 | (uint32_t)sb.i11 << 24;
+    }
+    q.sw[0][lane] = sb.w00;
+    q.sw[1][lane] = sb.w10;
+    q.sw[2][lane] = sb.w01;
+    q.sw[3][lane] = sb.w11;
+    return start;
+}
+
+__device__ __forceinline__ void store_rgba(const InferArgs &a, uint32_t r, f3 acc, float T)
+{
+    uint2 out;
+    out.x = (uint32_t)f2h(acc.x) | ((uint32_t)f2h(acc.y) << 16);
+    out.y = (uint32_t)f2h(acc.z) | ((uint32_t)f2h(1.0f - T) << 16);
+    reinterpret_cast<uint2 *>(a.rgba)[r] = out;
+}
+
+template <int RD, int RS, bool Q8, bool STATS, int MAP, int CHUNK, bool PACKED, bool QUADS>
+// 8 waves per SIMD need at most 64 VGPRs.  The fp16 kernel fits them; the q8
+// kernel spills 12 bytes per lane and is still faster than at 7 waves
+// (C4: 16.6 against 17.2 ms).  The statistics variants (tests and counters
+// only) keep their larger register budget.
+__global__ __launch_bounds__(INFER_BLOCK) __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 8)))
+void infer_kernel(InferArgs a, uint32_t total_slots)
+{
+    ShadeQueue &q = wave_queue<1>();
+    const int lane = (int)(threadIdx.x & 63u);
+    // every lane stays in the wave's loop to the end (it shades for others)
+    const uint32_t s = xcd_interleaved_block<INFER_XCD_CHUNK>() * blockDim.x + threadIdx.x;
+    const uint32_t r = s < total_slots ? slot_to_ray(a, s, MAP) : NONE;
+    bool active = r != NONE;
+    using Tex = typename std::conditional<Q8, TexQ8<RD, RS, QUADS>, TexF16<RD, RS, QUADS>>::type;
+    InferIntegrator<RD, RS, Tex> integ;
+    begin_integrator<Q8, QUADS>(integ, a);
     StatsAcc<STATS> st;
     st.begin(a.stats, r);
     typename std::conditional<PACKED, PackedWalk, WalkState>::type w;
     if (active) {
         uint32_t start;
-        if constexpr (MAP == MAP_CAMERA) {
-            // the ray of pixel (u, v) of image img, normalised as load_ray does
-            const uint32_t hw = a.H * a.W, img = r / hw, rem = r - img * hw, v = rem / a.W, u = rem - v * a.W;
-            f3 dd;
-            camera_ray(a.cams[img], u, v, a.H, integ.o, dd);
-            integ.d = divs(dd, __builtin_sqrtf(dot(dd, dd)));
-            start = a.start_point[a.start_rows ? img * a.H + v : img];
-        } else {
-            load_ray(a.rays, r, integ.o, integ.d);
-            start = a.start_point[a.rays_per_start ? r / a.rays_per_start : r];
-        }
-        float su, sv;
-        oct_encode<RS>(mk(-integ.d.x, -integ.d.y, -integ.d.z), su, sv);
-        Bilinear sb;
-        if constexpr (QUADS) {
-            sb = bilinear_quad<RS>(su, sv);
-            q.si[lane] = (uint32_t)sb.i00;
-        } else {
-            sb = bilinear_setup<RS>(su, sv);
-            q.si[lane] = (uint32_t)sb.i00 | (uint32_t)sb.i10 << 8 | (uint32_t)sb.i01 << 16 | (uint32_t)sb.i11 << 24;
-        }
-        q.sw[0][lane] = sb.w00;
-        q.sw[1][lane] = sb.w10;
-        q.sw[2][lane] = sb.w01;
-        q.sw[3][lane] = sb.w11;
+        start = begin_ray<RS, QUADS>(a, r, MAP == MAP_CAMERA, q, lane, integ.o, integ.d);
         if (start >= a.num_points) { // out of range: no step, rgba (0, 0, 0, 0)
             active = false;
             w.n = 0;
@@ -477,11 +507,71 @@ void infer_kernel(InferArgs a, uint32_t total_slots)
     }
     if (r == NONE)
         return;
-    uint2 out;
-    out.x = (uint32_t)f2h(integ.acc.x) | ((uint32_t)f2h(integ.acc.y) << 16);
-    out.y = (uint32_t)f2h(integ.acc.z) | ((uint32_t)f2h(1.0f - integ.T) << 16);
-    reinterpret_cast<uint2 *>(a.rgba)[r] = out;
+    store_rgba(a, r, integ.acc, integ.T);
     st.store(a.stats, r, w.n);
+}
+
+// The render with four lanes per ray (walk_step_group) over the scene's own
+// arrays, for launches of few tiles: the same images.
+template <int RD, int RS, bool Q8>
+__global__ __launch_bounds__(GROUP_BLOCK) void infer_group_kernel(InferArgs a, int map)
+{
+    __shared__ uint32_t most[2][GROUP_BLOCK / 64];
+    ShadeQueue &q = wave_queue<GROUP>();
+    const int lane = (int)(threadIdx.x & 63u);
+    const uint32_t tile = map != MAP_LINEAR && a.tile_order ? a.tile_order[blockIdx.x] : blockIdx.x;
+    const uint32_t s = tile * 64u + group_within(map != MAP_LINEAR && a.th == 8);
+    uint32_t r;
+    if (map != MAP_LINEAR) {
+        r = tiled_ray(s, a.num_images, a.H, a.W, a.th, a.tw);
+    } else {
+        r = s < a.num_rays ? a.ray_perm ? a.ray_perm[s] : s : NONE;
+        r = r < a.num_rays ? r : NONE;
+    }
+    bool active = r != NONE;
+    using Tex = typename std::conditional<Q8, TexQ8<RD, RS, false>, TexF16<RD, RS, false>>::type;
+    InferIntegrator<RD, RS, Tex, GROUP> integ;
+    begin_integrator<Q8, false>(integ, a);
+    StatsAcc<false> st;
+    GroupWalk w;
+    w.n = 0;
+    if (active) {
+        const uint32_t start = begin_ray<RS, false>(a, r, map == MAP_CAMERA, q, lane, integ.o, integ.d);
+        active = start < a.num_points; // out of range: no step, rgba (0, 0, 0, 0)
+        if (active)
+            group_begin(w, a.points, a.adjacency, a.offsets, a.adj_diff, start, (uint32_t)lane % GROUP);
+    }
+    q.mask[lane] = 0ull;
+    if (lane == 0)
+        q.tail = 0;
+    wave_lds_sync();
+    uint32_t head = 0; // wave-uniform: entries shaded so far
+    while (__ballot(active)) {
+        if (active)
+            active = walk_step_group(w, integ.o, integ.d, (uint32_t)lane % GROUP, a.points, a.adjacency, a.offsets,
+                                     a.adj_diff, a.max_steps, integ, st);
+        wave_lds_sync();
+        if (__builtin_amdgcn_readfirstlane(q.tail) - head >= 64u) {
+            shade_batch<RD, RS>(q, head, 64, integ, lane);
+            head += 64;
+        }
+    }
+    const uint32_t rest = __builtin_amdgcn_readfirstlane(q.tail) - head;
+    if (rest)
+        shade_batch<RD, RS>(q, head, rest, integ, lane);
+    if (map != MAP_LINEAR && a.tile_cost) {
+        const uint32_t nmax = wave_max_u32(w.n), fmax = wave_max_u32(st.face_count()), v = threadIdx.x >> 6;
+        if (lane == 0) {
+            most[0][v] = nmax;
+            most[1][v] = fmax;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0)
+            a.tile_cost[tile] = tile_cost_of(max(max(most[0][0], most[0][1]), max(most[0][2], most[0][3])),
+                                             max(max(most[1][0], most[1][1]), max(most[1][2], most[1][3])));
+    }
+    if (r != NONE && lane % GROUP == 0)
+        store_rgba(a, r, integ.acc, integ.T);
 }
 
 template <int RD, int RS, bool Q8, bool STATS, int MAP>
@@ -505,9 +595,22 @@ static int launch_one(const InferArgs &a, hipStream_t stream, uint32_t slots)
     return VT_OK;
 }
 
+// Launches of up to this many tiles (64 rays each) run with four lanes per ray
+// (see FWD_GROUP_TILES for why).  Heightfield scene of 300,000 sites, a render
+// with one wave per tile over the packed layout / with four over the scene's
+// arrays, us: 625 tiles 642 / 325, 1,024 tiles 642 / 373, 2,025 tiles 645 /
+// 627, 4,096 tiles 702 / 1,077.
+constexpr uint32_t INFER_GROUP_TILES = 1792;
+
 template <int RD, int RS, bool Q8>
 static int launch_infer_rs(const InferArgs &a, bool stats, int map, hipStream_t stream, uint32_t lanes)
 {
+    const uint32_t tiles = (lanes + 63) / 64;
+    if (!stats && tiles <= INFER_GROUP_TILES) {
+        infer_group_kernel<RD, RS, Q8><<<tiles, GROUP_BLOCK, 0, stream>>>(a, map);
+        VT_LAUNCH_CHECK("infer_group_kernel");
+        return VT_OK;
+    }
     if (map == MAP_CAMERA)
         return stats ? launch_one<RD, RS, Q8, true, MAP_CAMERA>(a, stream, lanes)
                      : launch_one<RD, RS, Q8, false, MAP_CAMERA>(a, stream, lanes);

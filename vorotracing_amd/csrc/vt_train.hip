@@ -76,7 +76,15 @@ template <typename A, int RD, int RS> struct TrainTex {
                            Attr<A>::load(m, b.i01 * 3 + c), Attr<A>::load(m, b.i11 * 3 + c));
         return mk(v[0], v[1], v[2]);
     }
-    // sigmoid(diffuse(probe) + specular(spec taps)); diffuse taps out in db
+    __device__ __forceinline__ static float sample_1(const A *__restrict__ m, const Bilinear &b, int c)
+    {
+        return bil_mix(b, Attr<A>::load(m, b.i00 * 3 + c), Attr<A>::load(m, b.i10 * 3 + c),
+                       Attr<A>::load(m, b.i01 * 3 + c), Attr<A>::load(m, b.i11 * 3 + c));
+    }
+    // sigmoid(diffuse(probe) + specular(spec taps)); diffuse taps out in db.
+    // G lanes per ray: each of the first three takes a channel (a third of the
+    // texel loads and sigmoids), and all get the three.
+    template <int G>
     __device__ __forceinline__ f3 color(uint32_t cell, f3 o, f3 d, float t0, f3 p, const Bilinear &spec,
                                         Bilinear &db) const
     {
@@ -84,6 +92,14 @@ template <typename A, int RD, int RS> struct TrainTex {
         float u, v;
         oct_encode<RD>(pd, u, v);
         db = bilinear_setup<RD>(u, v);
+        if constexpr (G > 1) {
+            static_assert(G == 4, "the broadcasts below are within quads");
+            const int g = (int)(threadIdx.x % G), c = g < 3 ? g : 2;
+            const uint32_t x =
+                f_bits(sigmoid(sample_1(diffuse + (size_t)cell * (3 * RD * RD), db, c) +
+                               sample_1(specular + (size_t)cell * (3 * RS * RS), spec, c)));
+            return mk(bits_f(quad_perm<0x00>(x)), bits_f(quad_perm<0x55>(x)), bits_f(quad_perm<0xaa>(x)));
+        }
         f3 a = sample(diffuse + (size_t)cell * (3 * RD * RD), db);
         f3 b = sample(specular + (size_t)cell * (3 * RS * RS), spec);
         f3 lg = add(a, b);
@@ -247,8 +263,9 @@ struct FwdArgs {
     uint32_t *tile_cost;        // tiled lane order: each tile's cost (tile_cost_of), or null
 };
 
-// RayIntegratorOctMap::integrate_cell (ray_integrator_octmap.cuh:102-152)
-template <typename A, int RD, int RS> struct FwdIntegrator {
+// RayIntegratorOctMap::integrate_cell (ray_integrator_octmap.cuh:102-152).
+// G: lanes per ray, of which the first adds to shared outputs.
+template <typename A, int RD, int RS, int G = 1> struct FwdIntegrator {
     f3 o, d;
     const float *__restrict__ density;
     TrainTex<A, RD, RS> tex;
@@ -305,7 +322,7 @@ template <typename A, int RD, int RS> struct FwdIntegrator {
         if (sig > 1e-6f) {
             st.shade();
             Bilinear db;
-            rgb = tex.color(cell, o, d, t0, p, spec, db);
+            rgb = tex.template color<G>(cell, o, d, t0, p, spec, db);
         }
         float dt = __builtin_fmaxf(t1 - t0, 0.0f);
         float alpha = 1.0f - vt_expf(-sig * dt);
@@ -322,7 +339,7 @@ template <typename A, int RD, int RS> struct FwdIntegrator {
         if (t1 > tfar)
             tfar = t1;
 
-        if (contribution)
+        if (contribution && (G == 1 || threadIdx.x % G == 0))
             scatter_contribution(cell, w);
         acc = vfma(w, rgb, acc);
 
@@ -344,10 +361,10 @@ template <typename A, int RD, int RS> struct FwdIntegrator {
 // hide more of the walk's load latency.
 // The forward of ray r; returns the walk's step count, and in faces the face
 // records it searched.
-template <typename A, int RD, int RS, bool STATS>
+template <typename A, int RD, int RS, bool STATS, int G = 1>
 __device__ __forceinline__ uint32_t fwd_ray(const FwdArgs &a, uint32_t r, uint32_t &faces)
 {
-    FwdIntegrator<A, RD, RS> it;
+    FwdIntegrator<A, RD, RS, G> it;
     load_ray(a.rays, r, it.o, it.d);
     it.density = a.density;
     it.tex.diffuse = (const A *)a.diffuse;
@@ -370,9 +387,16 @@ __device__ __forceinline__ uint32_t fwd_ray(const FwdArgs &a, uint32_t r, uint32
     StatsAcc<STATS> st;
     st.begin(a.stats, r);
     const uint32_t start = a.start_point[r];
-    const uint32_t n = start < a.num_points ? walk<TRAIN_CHUNK>(it.o, it.d, a.points, a.adjacency, a.offsets,
-                                                                a.adj_diff, start, a.max_steps, it, st)
-                                            : 0u;
+    uint32_t n = 0;
+    if (start < a.num_points) {
+        if constexpr (G == 1)
+            n = walk<TRAIN_CHUNK>(it.o, it.d, a.points, a.adjacency, a.offsets, a.adj_diff, start, a.max_steps, it, st);
+        else
+            n = walk_group(it.o, it.d, a.points, a.adjacency, a.offsets, a.adj_diff, start, a.max_steps, it, st);
+    }
+    faces = st.face_count();
+    if (G > 1 && threadIdx.x % G != 0)
+        return n; // the first lane writes
     for (uint32_t i = it.qi; i < K; ++i) {
         a.depth[(size_t)r * K + i] = -1.0f;
         a.depth_idx[(size_t)r * K + i] = NONE;
@@ -389,7 +413,6 @@ __device__ __forceinline__ uint32_t fwd_ray(const FwdArgs &a, uint32_t r, uint32
     a.S_total[r] = it.S;
     a.t_far[r] = it.tfar;
     st.store(a.stats, r, n);
-    faces = st.face_count();
     return n;
 }
 
@@ -418,6 +441,45 @@ void fwd_kernel(FwdArgs a)
                     a.tile_cost[t.tile] = tile_cost_of(nmax, fmax);
             }
         }
+    }
+}
+
+// The block's ray of a group launch (group_within), in the tile that its
+// place in the launch order has (tile NONE: past the last).
+__device__ __forceinline__ uint32_t group_ray(uint32_t num_rays, const uint32_t *perm, uint32_t ni, uint32_t h,
+                                              uint32_t w, const uint32_t *tile_order, uint32_t &tile)
+{
+    tile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
+    const bool tiled = ni && !perm;
+    const uint32_t q = tile * 64u + group_within(tiled);
+    if (tiled)
+        return tiled_ray<TRAIN_TILE_STRIP>(q, ni, h, w, TRAIN_TILE, TRAIN_TILE);
+    if (q >= num_rays)
+        return NONE;
+    const uint32_t r = perm ? perm[q] : q;
+    return r < num_rays ? r : NONE;
+}
+
+// The forward with four lanes per ray (walk_step_group), for launches of few
+// tiles.
+template <typename A, int RD, int RS>
+__global__ __launch_bounds__(GROUP_BLOCK) void fwd_group_kernel(FwdArgs a)
+{
+    __shared__ uint32_t most[2][GROUP_BLOCK / 64];
+    uint32_t tile, n = 0, faces = 0;
+    const uint32_t r = group_ray(a.num_rays, a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order, tile);
+    if (r != NONE)
+        n = fwd_ray<A, RD, RS, false, GROUP>(a, r, faces);
+    if (a.tile_cost && (a.num_images || a.ray_perm)) {
+        const uint32_t nmax = wave_max_u32(n), fmax = wave_max_u32(faces), w = threadIdx.x >> 6;
+        if ((threadIdx.x & 63u) == 0) {
+            most[0][w] = nmax;
+            most[1][w] = fmax;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0)
+            a.tile_cost[tile] = tile_cost_of(max(max(most[0][0], most[0][1]), max(most[0][2], most[0][3])),
+                                             max(max(most[1][0], most[1][1]), max(most[1][2], most[1][3])));
     }
 }
 
@@ -465,8 +527,10 @@ __device__ __forceinline__ f3 cell_intersection_grad(f3 prim, f3 opp, f3 o, f3 d
     return divs(g, dp * dp);
 }
 
-// RayIntegratorOctMapBackward::integrate_cell (ray_integrator_octmap.cuh:683-860)
-template <typename A, int RD, int RS> struct BwdIntegrator {
+// RayIntegratorOctMapBackward::integrate_cell (ray_integrator_octmap.cuh:683-860).
+// G: lanes per ray; the first of them is the ray's member of a group (its row
+// holds the record), and all of them work on the columns.
+template <typename A, int RD, int RS, int G = 1> struct BwdIntegrator {
     f3 o, d;
     const float *__restrict__ density;
     TrainTex<A, RD, RS> tex;
@@ -688,6 +752,12 @@ template <typename A, int RD, int RS> struct BwdIntegrator {
     // lanes, groups of a single lane are set aside and sent two per pass
     // afterwards: lanes of rank k < REC_COLS send column k of the first,
     // lanes of rank REC_COLS + k column k of the second.
+    __device__ __forceinline__ static uint64_t members(uint64_t act)
+    {
+        static_assert(G == 1 || G == 4, "the mask below takes every G-th lane");
+        return G == 1 ? act : act & 0x1111111111111111ull;
+    }
+
     template <bool ONE>
     __device__ __forceinline__ void combine(uint32_t cell, uint64_t act, uint32_t nact, uint32_t arank, uint32_t lane)
     {
@@ -696,7 +766,7 @@ template <typename A, int RD, int RS> struct BwdIntegrator {
         Column c1;
         if (ONE)
             c1 = column(arank - half * (uint32_t)REC_COLS);
-        uint64_t pend = act, singles = 0;
+        uint64_t pend = members(act), singles = 0;
         while (pend) { // one group per pass, at most 64
             const int ll = (int)__builtin_ctzll(pend);
             const uint32_t lead = __builtin_amdgcn_readlane(cell, ll);
@@ -751,7 +821,7 @@ template <typename A, int RD, int RS> struct BwdIntegrator {
     {
         const bool color = held_taps != HELD_NO_COLOR;
         const uint32_t lane = threadIdx.x & 63u;
-        {
+        if (G == 1 || lane % G == 0) {
             float4 *row = reinterpret_cast<float4 *>(rows + lane * ROW_STRIDE);
             const float g0 = color ? held_gl[0] : 0.0f, g1 = color ? held_gl[1] : 0.0f,
                         g2 = color ? held_gl[2] : 0.0f;
@@ -797,7 +867,7 @@ template <typename A, int RD, int RS> struct BwdIntegrator {
         bool has_color = false;
         if (sig > 1e-6f) {
             st.shade();
-            rgb = tex.color(cell, o, d, t0, p, spec, db);
+            rgb = tex.template color<G>(cell, o, d, t0, p, spec, db);
             has_color = true;
         }
         float dt = __builtin_fmaxf(t1 - t0, 0.0f);
@@ -896,20 +966,11 @@ template <typename A, int RD, int RS> struct BwdIntegrator {
     }
 };
 
-template <typename A, int RD, int RS, bool STATS>
-__global__ __launch_bounds__(TRAIN_BLOCK) __attribute__((amdgpu_waves_per_eu(TRAIN_BWD_WAVES)))
-void bwd_kernel(BwdArgs a)
+// The backward of ray r; rows: the wave's LDS row table.
+template <typename A, int RD, int RS, bool STATS, int G = 1>
+__device__ __forceinline__ void bwd_ray(const BwdArgs &a, uint32_t r, float *rows)
 {
-    __shared__ __align__(16) float rows_lds[TRAIN_WAVES][ROW_TABLE_FLOATS];
-    float *rows = rows_lds[threadIdx.x / 64];
-    if ((threadIdx.x & 63u) < (uint32_t)ROW_STRIDE)
-        rows[64 * ROW_STRIDE + (threadIdx.x & 63u)] = 0.0f; // the zero row
-    wave_lds_sync();
-    uint32_t r = train_ray<false>(xcd_interleaved_block<TRAIN_XCD_CHUNK>() * blockDim.x + threadIdx.x, a.num_rays,
-                                  a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order);
-    if (r == NONE)
-        return;
-    BwdIntegrator<A, RD, RS> it;
+    BwdIntegrator<A, RD, RS, G> it;
     it.rows = rows;
     load_ray(a.rays, r, it.o, it.d);
     it.density = a.density;
@@ -968,12 +1029,53 @@ void bwd_kernel(BwdArgs a)
     StatsAcc<STATS> st;
     st.begin(a.stats, r);
     const uint32_t start = a.start_point[r];
-    const uint32_t n = start < a.num_points ? walk<TRAIN_BWD_CHUNK>(it.o, it.d, a.points, a.adjacency, a.offsets,
-                                                                    a.adj_diff, start, a.max_steps, it, st)
-                                            : 0u;
+    uint32_t n = 0;
+    if (start < a.num_points) {
+        if constexpr (G == 1)
+            n = walk<TRAIN_BWD_CHUNK>(it.o, it.d, a.points, a.adjacency, a.offsets, a.adj_diff, start, a.max_steps, it,
+                                      st);
+        else
+            n = walk_group(it.o, it.d, a.points, a.adjacency, a.offsets, a.adj_diff, start, a.max_steps, it, st);
+    }
     it.finish();
     st.store(a.stats, r, n);
 }
+
+// The zero row of a wave's table.
+__device__ __forceinline__ float *begin_rows(float *rows)
+{
+    if ((threadIdx.x & 63u) < (uint32_t)ROW_STRIDE)
+        rows[64 * ROW_STRIDE + (threadIdx.x & 63u)] = 0.0f;
+    wave_lds_sync();
+    return rows;
+}
+
+template <typename A, int RD, int RS, bool STATS>
+__global__ __launch_bounds__(TRAIN_BLOCK) __attribute__((amdgpu_waves_per_eu(TRAIN_BWD_WAVES)))
+void bwd_kernel(BwdArgs a)
+{
+    __shared__ __align__(16) float rows_lds[TRAIN_WAVES][ROW_TABLE_FLOATS];
+    float *rows = begin_rows(rows_lds[threadIdx.x / 64]);
+    const uint32_t r = train_ray<false>(xcd_interleaved_block<TRAIN_XCD_CHUNK>() * blockDim.x + threadIdx.x,
+                                        a.num_rays, a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order);
+    if (r != NONE)
+        bwd_ray<A, RD, RS, STATS>(a, r, rows);
+}
+
+// The backward with four lanes per ray, for launches of few tiles: besides the
+// face search, the combining rounds of a wave-step get fewer (16 rays meet
+// fewer cells than 64).
+template <typename A, int RD, int RS>
+__global__ __launch_bounds__(GROUP_BLOCK) void bwd_group_kernel(BwdArgs a)
+{
+    __shared__ __align__(16) float rows_lds[GROUP_BLOCK / 64][ROW_TABLE_FLOATS];
+    float *rows = begin_rows(rows_lds[threadIdx.x / 64]);
+    uint32_t tile;
+    const uint32_t r = group_ray(a.num_rays, a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order, tile);
+    if (r != NONE)
+        bwd_ray<A, RD, RS, false, GROUP>(a, r, rows);
+}
+
 
 int prefetch(const float *points, uint32_t num_points, const uint32_t *adjacency, uint32_t adjacency_size,
              const uint32_t *offsets, uint16_t *adj_diff, hipStream_t stream);
@@ -1003,18 +1105,47 @@ static uint32_t resident_waves(uint32_t waves_per_simd)
     return (uint32_t)cus * 4u * waves_per_simd;
 }
 
+// Launches of up to this many tiles (64 rays each) run with four lanes per ray.
+// One wave per tile leaves the chip's 1,024 SIMDs a wave or two each and lasts
+// as long as its longest wave whatever their number; four waves per tile fill
+// it, and lose once they no longer fit at once.  Torus scene of 131,072 sites,
+// entry times in us with a wave per tile / four:
+//   tiles      1,024        2,025        3,025        4,096
+//   forward    858 / 530    842 / 678    870 / 811    939 / 1,011
+//   backward  2,381 / 1,280  2,459 / 1,520             2,432 / 2,540
+// (heightfield, 2,025 tiles: forward 606 / 615, backward 1,376 / 1,350).
+constexpr uint32_t FWD_GROUP_TILES = 1792, BWD_GROUP_TILES = 3072;
+
+template <typename A> constexpr bool F16 = std::is_same<A, uint16_t>::value;
+
 template <typename A, int RD, int RS, bool ST> struct FwdK {
     static constexpr auto fn = fwd_kernel<A, RD, RS, ST>;
+    static constexpr auto group_fn = fwd_group_kernel<A, RD, RS>;
+    // (a contribution in half storage keeps the wave's larger sums: below)
+    static uint32_t group_tiles(const FwdArgs &a) { return F16<A> && a.contribution ? 0u : FWD_GROUP_TILES; }
     static uint32_t resident() { return resident_waves(TRAIN_FWD_WAVES); }
 };
 template <typename A, int RD, int RS, bool ST> struct BwdK {
     static constexpr auto fn = bwd_kernel<A, RD, RS, ST>;
+    static constexpr auto group_fn = bwd_group_kernel<A, RD, RS>;
+    // 16 rays of a wave meet in fewer f32 sums than 64, so half gradients
+    // would be rounded more often (their error against 64 bits 0.0028 with a
+    // wave per tile, 0.0040 with four)
+    static uint32_t group_tiles(const BwdArgs &) { return F16<A> ? 0u : BWD_GROUP_TILES; }
     static uint32_t resident() { return resident_waves(TRAIN_BWD_WAVES); }
 };
 
 template <template <typename, int, int, bool> class K, typename Args, typename A, int RD, int RS>
 static int launch_train_rs(const Args &a, bool stats, hipStream_t s)
 {
+    using Kernel = K<A, RD, RS, false>;
+    const uint64_t all = a.num_images && !a.ray_perm ? train_tiles(a.num_rays, false, a.num_images, a.img_h, a.img_w)
+                                                     : ((uint64_t)a.num_rays + 63) / 64;
+    if (!stats && all <= Kernel::group_tiles(a)) {
+        hipLaunchKernelGGL((Kernel::group_fn), dim3((uint32_t)all), dim3(GROUP_BLOCK), 0, s, a);
+        VT_LAUNCH_CHECK("training traversal kernel (four lanes per ray)");
+        return VT_OK;
+    }
     uint64_t slots = a.num_rays;
     if (a.num_images || a.ray_perm) {
         const uint64_t tiles = train_tiles(a.num_rays, a.ray_perm != nullptr, a.num_images, a.img_h, a.img_w);

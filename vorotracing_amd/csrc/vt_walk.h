@@ -214,6 +214,204 @@ __device__ __forceinline__ uint32_t walk(f3 o, f3 d, const float *points,
 }
 
 // ---------------------------------------------------------------------------
+// The same walk with GROUP lanes of a wave per ray, for launches that leave
+// most of the chip idle: with a wave per 64 rays such a launch lasts as long
+// as one wave's chain of loads and face searches (16,384 rays are 256 waves
+// on 1,024 SIMDs).  Lane g of a ray's quad searches the faces j = g (mod 4),
+// the four candidates meet by two DPP steps, and everything else is computed
+// alike in all four lanes.  Each lane's neighbour ids come with its face
+// records, and the next cell's records are loaded before the integrator runs,
+// so a step waits for two loads after one another instead of three, and the
+// second behind the integrator's work.  16,384 rays over 4,096 sites: the
+// training forward's entry 289 -> 170 us, its backward's 715 -> 410.
+constexpr int GROUP = 4;
+constexpr int GROUP_CHUNK = 6; // faces per lane and pass: 24 of a cell's 16 or so at once
+
+template <int CTRL> __device__ __forceinline__ uint32_t quad_perm(uint32_t x)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+}
+
+struct GroupWalk {
+    uint32_t cur;
+    f3 p;
+    float t0;
+    uint32_t n;
+    uint32_t b, nf;                // face list
+    uint2 rec[GROUP_CHUNK];        // the lane's first faces g, g + 4, ...
+    uint32_t nbr[GROUP_CHUNK];     // and the neighbours behind them
+};
+
+// The lane's faces [GROUP * first + g, ...) of the list of nf at b.  Records
+// past its end stay inside the 32-row padding; neighbour ids, whose array has
+// no padding of its own, are read for faces of the list only.
+__device__ __forceinline__ void group_load(const uint2 *adj_diff, const uint32_t *adjacency, uint32_t b, uint32_t nf,
+                                           uint32_t first, uint32_t g, uint2 *rec, uint32_t *nbr)
+{
+    static_assert(GROUP * GROUP_CHUNK <= 32, "reads past a list end must stay inside the 32-row padding");
+#pragma unroll
+    for (int s = 0; s < GROUP_CHUNK; ++s)
+        rec[s] = adj_diff[b + first + GROUP * s + g];
+#pragma unroll
+    for (int s = 0; s < GROUP_CHUNK; ++s) {
+        nbr[s] = NONE;
+        if (first + GROUP * s + g < nf)
+            nbr[s] = adjacency[b + first + GROUP * s + g];
+    }
+}
+
+__device__ __forceinline__ void group_begin(GroupWalk &w, const float *points, const uint32_t *adjacency,
+                                            const uint32_t *offsets, const uint2 *adj_diff, uint32_t start, uint32_t g)
+{
+    w.cur = start;
+    w.p = load_site(points, start);
+    w.b = offsets[start];
+    w.nf = offsets[start + 1] - w.b;
+    w.t0 = 0.0f;
+    w.n = 0;
+    group_load(adj_diff, adjacency, w.b, w.nf, 0, g, w.rec, w.nbr);
+}
+
+// exit_face over the four lanes of a quad: every lane gets the face of the
+// lowest quotient, ties to the lowest index, its t1 and the neighbour behind
+// it (nxt).  A lane's own search is exit_face's over its faces, so its best is
+// the first of its lowest IEEE quotients, and the quotients themselves are
+// compared between lanes.
+__device__ __forceinline__ uint32_t group_exit_face(const GroupWalk &w, const uint2 *adj_diff,
+                                                    const uint32_t *adjacency, f3 o, f3 d, uint32_t g, float &t1,
+                                                    uint32_t &nxt)
+{
+    const f3 p = w.p;
+    uint32_t best = NONE, nb = NONE;
+    float bnum = FIRST_BNUM, bdp = FIRST_BDP;
+    uint2 rec[GROUP_CHUNK];
+    uint32_t nbr[GROUP_CHUNK];
+#pragma unroll
+    for (int s = 0; s < GROUP_CHUNK; ++s) {
+        rec[s] = w.rec[s];
+        nbr[s] = w.nbr[s];
+    }
+    for (uint32_t first = 0;;) {
+#pragma unroll
+        for (int s = 0; s < GROUP_CHUNK; ++s) {
+            // as in exit_face: keep the widening out of v_fma_mix operands
+            float ox = half_lo(rec[s].x), oy = half_hi(rec[s].x), oz = half_lo(rec[s].y);
+            asm("" : "+v"(ox), "+v"(oy), "+v"(oz));
+            const float dp = fma_(oz, d.z, fma_(oy, d.y, ox * d.x));
+            const uint32_t j = first + GROUP * s + g;
+            if (dp > 0.0f && j < w.nf) {
+                const float ex = fma_(ox, 0.5f, p.x) - o.x;
+                const float ey = fma_(oy, 0.5f, p.y) - o.y;
+                const float ez = fma_(oz, 0.5f, p.z) - o.z;
+                const float num = fma_(ez, oz, fma_(ey, oy, ex * ox));
+                if (exit_before(num, dp, bnum, bdp)) {
+                    bnum = num;
+                    bdp = dp;
+                    best = j;
+                    nb = nbr[s];
+                }
+            }
+        }
+        first += GROUP * GROUP_CHUNK;
+        if (first >= w.nf) // (the same in the four lanes)
+            break;
+        group_load(adj_diff, adjacency, w.b, w.nf, first, g, rec, nbr);
+    }
+    float t = __builtin_huge_valf();
+    if (best != NONE)
+        t = bnum / bdp;
+    if (t == -__builtin_huge_valf()) { // see exit_face
+        float bt = __builtin_huge_valf();
+        for (uint32_t j = g; j < w.nf; j += GROUP) {
+            float num, dp;
+            face_terms(adj_diff[w.b + j], p, o, d, num, dp);
+            if (dp > 0.0f) {
+                const float q = num / dp;
+                if (q < bt) {
+                    bt = q;
+                    best = j;
+                    nb = adjacency[w.b + j];
+                }
+            }
+        }
+        t = bt;
+    }
+#define VT_GROUP_MEET(CTRL)                                                                                           \
+    {                                                                                                                 \
+        const float ot = bits_f(quad_perm<CTRL>(f_bits(t)));                                                          \
+        const uint32_t ob = quad_perm<CTRL>(best), on = quad_perm<CTRL>(nb);                                          \
+        const bool take = ot < t || (ot == t && ob < best);                                                           \
+        t = take ? ot : t;                                                                                            \
+        best = take ? ob : best;                                                                                      \
+        nb = take ? on : nb;                                                                                          \
+    }
+    VT_GROUP_MEET(0xb1) // lanes 1, 0, 3, 2
+    VT_GROUP_MEET(0x4e) // lanes 2, 3, 0, 1
+#undef VT_GROUP_MEET
+    t1 = t;
+    nxt = nb;
+    return best;
+}
+
+// walk_step for a quad (the same in its four lanes, g apart).
+template <class Integrator, class StatsT>
+__device__ __forceinline__ bool walk_step_group(GroupWalk &w, f3 o, f3 d, uint32_t g, const float *points,
+                                                const uint32_t *adjacency, const uint32_t *offsets,
+                                                const uint2 *adj_diff, uint32_t max_steps, Integrator &integ,
+                                                StatsT &st)
+{
+    w.n++;
+    if (w.n > max_steps)
+        return false;
+    integ.begin_cell(w.cur);
+    st.visit(w.cur, w.nf);
+    float t1;
+    uint32_t nxt;
+    if (group_exit_face(w, adj_diff, adjacency, o, d, g, t1, nxt) == NONE)
+        return false;
+    st.exit();
+    const f3 p = w.p, np = load_site(points, nxt);
+    const uint32_t cur = w.cur;
+    w.b = offsets[nxt];
+    w.nf = offsets[nxt + 1] - w.b;
+    group_load(adj_diff, adjacency, w.b, w.nf, 0, g, w.rec, w.nbr);
+    // no early return inside the integrate branch (see walk_step)
+    bool go = true;
+    if (t1 > w.t0) {
+        st.integrate();
+        go = integ.integrate(cur, w.t0, t1, p, np, st);
+    }
+    w.t0 = __builtin_fmaxf(w.t0, t1);
+    w.cur = nxt;
+    w.p = np;
+    return go;
+}
+
+// walk for a quad.
+template <class Integrator, class StatsT>
+__device__ __forceinline__ uint32_t walk_group(f3 o, f3 d, const float *points, const uint32_t *adjacency,
+                                               const uint32_t *offsets, const uint2 *adj_diff, uint32_t start,
+                                               uint32_t max_steps, Integrator &integ, StatsT &st)
+{
+    const uint32_t g = threadIdx.x % GROUP;
+    GroupWalk w;
+    group_begin(w, points, adjacency, offsets, adj_diff, start, g);
+    while (walk_step_group(w, o, d, g, points, adjacency, offsets, adj_diff, max_steps, integ, st)) {
+    }
+    return w.n;
+}
+
+// The rays of a group launch: a block of four waves per 8x8 screen tile or 64
+// rays in a row, 16 of them to a wave (a 4x4 quarter of a tile), four lanes
+// each.  Returns the ray's place among the block's 64.
+constexpr int GROUP_BLOCK = 64 * GROUP;
+__device__ __forceinline__ uint32_t group_within(bool tiled)
+{
+    const uint32_t w = threadIdx.x >> 6, i = (threadIdx.x & 63u) / GROUP;
+    return tiled ? ((w >> 1) * 4u + (i >> 2)) * 8u + (w & 1u) * 4u + (i & 3u) : w * 16u + i;
+}
+
+// ---------------------------------------------------------------------------
 // The same walk over the packed walk layout (vt_walk_layout, built by
 // vt_walk_layout_fill).  The traversal kernels are bound by the number of
 // vector memory instructions they issue, so the layout regroups the scene's
