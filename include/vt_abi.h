@@ -30,7 +30,10 @@ enum {
     VT_ERR_NOMEM = 4
 };
 
-enum { VT_ATTR_F32 = 0, VT_ATTR_F16 = 1 };
+/* VT_ATTR_F16_SUMS (vt_trace_bwd only): half attributes whose texture
+ * gradients are summed in f32 and rounded once, where VT_ATTR_F16 adds halves
+ * and rounds at every addition; cell_workspace is larger then. */
+enum { VT_ATTR_F32 = 0, VT_ATTR_F16 = 1, VT_ATTR_F16_SUMS = 2 };
 
 /* Per-ray walk statistics (debug / roofline accounting).  Filled only when a
  * non-NULL `stats` array (one record per ray, in ray order) is passed.  The
@@ -364,7 +367,8 @@ int vt_trace_fwd(int attr_dtype, const float *points, const void *diffuse, const
  *   diffuse_grad / specular_grad attr dtype, density_grad f32 (num_points),
  *   point_error attr dtype (num_points) or NULL.
  *   image_h, image_w, ray_perm: lane order, as for vt_trace_fwd.
- *   cell_workspace: f32 (num_points, 4), 16-byte aligned, any contents (an
+ *   cell_workspace: f32 (num_points, 4), for VT_ATTR_F16_SUMS num_points * (4
+ *   + 3 diff_res^2 + 3 spec_res^2) floats, 16-byte aligned, any contents (an
  *   extension, ABI version 4): the call accumulates each cell's point and
  *   density gradients there, in one 16-byte slot per cell, and adds the
  *   slots into points_grad and density_grad at its end.

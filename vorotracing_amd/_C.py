@@ -681,7 +681,10 @@ def trace_vorotracing_bwd(points_in, diffuse_in, specular_in, density_in, point_
     points_grad = torch.zeros((num_points, 3), dtype=rays.dtype, device=dev)
     ray_grad = torch.zeros_like(rays)
     workspace = _adj_diff_buffer(adj_diff, adjacency_size, dev, "adj_diff")
-    cell_workspace = torch.empty((num_points, 4), dtype=torch.float32, device=dev)
+    # half maps: their gradients are summed in f32, behind the cells' slots, and rounded once
+    sums = diffuse.numel() + specular.numel() if code == 1 else 0
+    cell_workspace = torch.empty(4 * num_points + sums, dtype=torch.float32, device=dev)
+    code = 2 if code == 1 else code
     img_h, img_w, perm = _lane_order(rays, start_point, num_points, ray_perm)
     with torch.cuda.device(dev):
         sch, frame = _train_schedule(rays_in, img_h, img_w, num_rays, perm, ray_perm, dev)

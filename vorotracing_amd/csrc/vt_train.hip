@@ -529,8 +529,9 @@ __device__ __forceinline__ f3 cell_intersection_grad(f3 prim, f3 opp, f3 o, f3 d
 
 // RayIntegratorOctMapBackward::integrate_cell (ray_integrator_octmap.cuh:683-860).
 // G: lanes per ray; the first of them is the ray's member of a group (its row
-// holds the record), and all of them work on the columns.
-template <typename A, int RD, int RS, int G = 1> struct BwdIntegrator {
+// holds the record), and all of them work on the columns.  GA: storage of the
+// texture gradients, A or float (VT_ATTR_F16_SUMS).
+template <typename A, int RD, int RS, int G = 1, typename GA = A> struct BwdIntegrator {
     f3 o, d;
     const float *__restrict__ density;
     TrainTex<A, RD, RS> tex;
@@ -543,7 +544,8 @@ template <typename A, int RD, int RS, int G = 1> struct BwdIntegrator {
     float qval;
     const float *qthr, *depth_grad;
     float *cell_grad; // per cell (point gradient x, y, z, density gradient)
-    A *diffuse_grad, *specular_grad, *point_error;
+    GA *diffuse_grad, *specular_grad;
+    A *point_error;
     f3 prev_geom, prev_grad, cur_grad, next_grad;
     uint32_t prev_idx;
     f3 fwd_rgb, fwd_rgb_grad;
@@ -592,7 +594,7 @@ template <typename A, int RD, int RS, int G = 1> struct BwdIntegrator {
     struct Column {
         uint32_t k, sh, tmask;
         bool diffuse_taps, on;
-        bool attr; // the target holds attribute values (textures, point_error), else f32
+        bool attr; // the target holds half values (textures, point_error), else f32
         void *base;
         uint32_t stride, off, taps; // taps: texels of the map (1 for other columns)
     };
@@ -607,7 +609,7 @@ template <typename A, int RD, int RS, int G = 1> struct BwdIntegrator {
         c.diffuse_taps = k < 12u;
         c.on = k != 25u || point_error;
         c.taps = k < 12u ? RD * RD : k < 24u ? RS * RS : 1u;
-        c.attr = k < 24u || k == 25u;
+        c.attr = !std::is_same<A, float>::value && (k < 24u ? !std::is_same<GA, float>::value : k == 25u);
         c.base = k < 12u    ? static_cast<void *>(diffuse_grad)
                  : k < 24u  ? static_cast<void *>(specular_grad)
                  : k == 25u ? static_cast<void *>(point_error)
@@ -654,6 +656,11 @@ template <typename A, int RD, int RS, int G = 1> struct BwdIntegrator {
         if constexpr (std::is_same<A, float>::value) {
             if (send)
                 atomicAdd(static_cast<float *>(c.base) + i, x);
+        } else if constexpr (std::is_same<GA, float>::value) {
+            if (send && !c.attr)
+                atomicAdd(static_cast<float *>(c.base) + i, x);
+            else if (send) // point_error
+                Attr<A>::add(static_cast<A *>(c.base), i, x);
         } else {
             if (!c.attr) {
                 if (send)
@@ -967,10 +974,10 @@ template <typename A, int RD, int RS, int G = 1> struct BwdIntegrator {
 };
 
 // The backward of ray r; rows: the wave's LDS row table.
-template <typename A, int RD, int RS, bool STATS, int G = 1>
+template <typename A, int RD, int RS, bool STATS, int G = 1, typename GA = A>
 __device__ __forceinline__ void bwd_ray(const BwdArgs &a, uint32_t r, float *rows)
 {
-    BwdIntegrator<A, RD, RS, G> it;
+    BwdIntegrator<A, RD, RS, G, GA> it;
     it.rows = rows;
     load_ray(a.rays, r, it.o, it.d);
     it.density = a.density;
@@ -1011,8 +1018,8 @@ __device__ __forceinline__ void bwd_ray(const BwdArgs &a, uint32_t r, float *row
     it.depth_grad = K ? a.depth_grad + (size_t)r * K : nullptr;
     it.qval = K ? it.qthr[0] : 0.0f;
     it.cell_grad = a.cell_grad;
-    it.diffuse_grad = (A *)a.diffuse_grad;
-    it.specular_grad = (A *)a.specular_grad;
+    it.diffuse_grad = (GA *)a.diffuse_grad;
+    it.specular_grad = (GA *)a.specular_grad;
     it.point_error = (A *)a.point_error;
     it.prev_geom = it.prev_grad = it.cur_grad = it.next_grad = mk(0.0f, 0.0f, 0.0f);
     it.prev_idx = NONE;
@@ -1050,7 +1057,7 @@ __device__ __forceinline__ float *begin_rows(float *rows)
     return rows;
 }
 
-template <typename A, int RD, int RS, bool STATS>
+template <typename A, int RD, int RS, bool STATS, typename GA = A>
 __global__ __launch_bounds__(TRAIN_BLOCK) __attribute__((amdgpu_waves_per_eu(TRAIN_BWD_WAVES)))
 void bwd_kernel(BwdArgs a)
 {
@@ -1059,13 +1066,13 @@ void bwd_kernel(BwdArgs a)
     const uint32_t r = train_ray<false>(xcd_interleaved_block<TRAIN_XCD_CHUNK>() * blockDim.x + threadIdx.x,
                                         a.num_rays, a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order);
     if (r != NONE)
-        bwd_ray<A, RD, RS, STATS>(a, r, rows);
+        bwd_ray<A, RD, RS, STATS, 1, GA>(a, r, rows);
 }
 
 // The backward with four lanes per ray, for launches of few tiles: besides the
 // face search, the combining rounds of a wave-step get fewer (16 rays meet
 // fewer cells than 64).
-template <typename A, int RD, int RS>
+template <typename A, int RD, int RS, typename GA = A>
 __global__ __launch_bounds__(GROUP_BLOCK) void bwd_group_kernel(BwdArgs a)
 {
     __shared__ __align__(16) float rows_lds[GROUP_BLOCK / 64][ROW_TABLE_FLOATS];
@@ -1073,7 +1080,7 @@ __global__ __launch_bounds__(GROUP_BLOCK) void bwd_group_kernel(BwdArgs a)
     uint32_t tile;
     const uint32_t r = group_ray(a.num_rays, a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order, tile);
     if (r != NONE)
-        bwd_ray<A, RD, RS, false, GROUP>(a, r, rows);
+        bwd_ray<A, RD, RS, false, GROUP, GA>(a, r, rows);
 }
 
 
@@ -1127,11 +1134,21 @@ template <typename A, int RD, int RS, bool ST> struct FwdK {
 };
 template <typename A, int RD, int RS, bool ST> struct BwdK {
     static constexpr auto fn = bwd_kernel<A, RD, RS, ST>;
-    static constexpr auto group_fn = bwd_group_kernel<A, RD, RS>;
+    static constexpr auto group_fn = bwd_group_kernel<float, RD, RS>; // (f32: below)
     // 16 rays of a wave meet in fewer f32 sums than 64, so half gradients
     // would be rounded more often (their error against 64 bits 0.0028 with a
     // wave per tile, 0.0040 with four)
     static uint32_t group_tiles(const BwdArgs &) { return F16<A> ? 0u : BWD_GROUP_TILES; }
+    static uint32_t resident() { return resident_waves(TRAIN_BWD_WAVES); }
+};
+// Half attributes whose texture gradients are summed in f32: f32 atomics in
+// place of the packed half ones, each gradient rounded once.  121,512 rays over
+// 131,072 sites, a step: 4,296 -> 2,610 us, the gradients' error against 64
+// bits 0.0030 -> 0.0008.
+template <typename A, int RD, int RS, bool ST> struct BwdSumsK {
+    static constexpr auto fn = bwd_kernel<uint16_t, RD, RS, ST, float>;
+    static constexpr auto group_fn = bwd_group_kernel<uint16_t, RD, RS, float>;
+    static uint32_t group_tiles(const BwdArgs &a) { return a.point_error ? 0u : BWD_GROUP_TILES; }
     static uint32_t resident() { return resident_waves(TRAIN_BWD_WAVES); }
 };
 
@@ -1279,6 +1296,22 @@ __global__ void cell_grad_out_kernel(const float4 *g, float *points_grad, float 
     }
 }
 
+// Half gradients from their f32 sums: one rounding each (the outputs are
+// zero-initialised by the caller, as for the atomics).
+__global__ void attr_sums_clear_kernel(float *sums, size_t n)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        sums[i] = 0.0f;
+}
+
+__global__ void attr_sums_out_kernel(const float *sums, uint16_t *grad, size_t n)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        grad[i] = f2h(h2f(grad[i]) + sums[i]);
+}
+
 extern "C" int vt_trace_bwd(int attr_dtype, const float *points, const void *diffuse, const void *specular,
                             uint32_t diff_res, uint32_t spec_res, const float *density, const uint32_t *adjacency,
                             uint32_t adjacency_size, const uint32_t *offsets, uint32_t num_points, const float *rays,
@@ -1350,9 +1383,24 @@ extern "C" int vt_trace_bwd(int attr_dtype, const float *points, const void *dif
     const uint32_t cblocks = (num_points + 255) / 256;
     cell_grad_clear_kernel<<<cblocks, 256, 0, s>>>(reinterpret_cast<float4 *>(cell_workspace), num_points);
     VT_LAUNCH_CHECK("cell_grad_clear_kernel");
-    rc = launch_train<BwdK>(attr_dtype, a, diff_res, spec_res, stats != nullptr, s);
-    if (rc)
-        return rc;
+    const size_t nd = (size_t)num_points * 3 * diff_res * diff_res, ns = (size_t)num_points * 3 * spec_res * spec_res;
+    if (attr_dtype == VT_ATTR_F16_SUMS) {
+        float *attr_sums = cell_workspace + 4 * (size_t)num_points;
+        a.diffuse_grad = attr_sums;
+        a.specular_grad = attr_sums + nd;
+        attr_sums_clear_kernel<<<(uint32_t)((nd + ns + 255) / 256), 256, 0, s>>>(attr_sums, nd + ns);
+        VT_LAUNCH_CHECK("attr_sums_clear_kernel");
+        rc = launch_train_a<BwdSumsK, BwdArgs, uint16_t>(a, diff_res, spec_res, stats != nullptr, s);
+        if (rc)
+            return rc;
+        attr_sums_out_kernel<<<(uint32_t)((nd + 255) / 256), 256, 0, s>>>(attr_sums, (uint16_t *)diffuse_grad, nd);
+        attr_sums_out_kernel<<<(uint32_t)((ns + 255) / 256), 256, 0, s>>>(attr_sums + nd, (uint16_t *)specular_grad, ns);
+        VT_LAUNCH_CHECK("attr_sums_out_kernel");
+    } else {
+        rc = launch_train<BwdK>(attr_dtype, a, diff_res, spec_res, stats != nullptr, s);
+        if (rc)
+            return rc;
+    }
     cell_grad_out_kernel<<<cblocks, 256, 0, s>>>(reinterpret_cast<const float4 *>(cell_workspace), points_grad,
                                                   density_grad, num_points);
     VT_LAUNCH_CHECK("cell_grad_out_kernel");
