@@ -570,7 +570,7 @@ def voronoi_c3(sc, dev, log, reps=5):
                                                                qadj[np.lexsort((qadj, rows))]))
     out = {"sites": int(pts.shape[0]), "faces": int(off[-1]), "ms": round(1000 * float(np.median(times)), 1),
            "ms_min": round(1000 * min(times), 1), "equal_to_qhull": equal,
-           "note": "wall time of build_voronoi_adjacency (grid bucketing, cell clipping, CSR), median of "
+           "note": "wall time of build_voronoi_adjacency (site tree, cell clipping, CSR), median of "
                    f"{reps}; sets compared with scipy/qhull Delaunay.vertex_neighbor_vertices"}
     if "build_s" in sc.params:
         out["host_qhull_scene_s"] = sc.params["build_s"]
