@@ -145,6 +145,21 @@ def test_cell_with_many_faces(gpu, faces):
     _check(pts, gpu)
 
 
+@pytest.mark.parametrize("e", [-125, -100, -70, -40, -20, 30, 44, 60, 64, 90, 125])
+def test_any_unit(gpu, e):
+    """Sites times 2^e have the neighbours that they have at 1, lists of more
+    than a wave's vertices among them (squares of such coordinates leave f32),
+    in a cold build and from the neighbours at 1."""
+    pts = np.unique(np.round(H.mini_heightfield().points[::4] * 2.0 ** 20) / 2.0 ** 20, axis=0).astype(np.float32)
+    ref = ops.build_voronoi_adjacency(H.to_dev(pts, gpu))
+    far = np.ldexp(pts, e).astype(np.float32)
+    assert np.array_equal(np.ldexp(far.astype(np.float64), -e), pts), "a coordinate lost bits"
+    guesses = dict(initial_guesses=ref[0], initial_guesses_offsets=ref[1])
+    for kw in ({}, guesses):
+        got = ops.build_voronoi_adjacency(H.to_dev(far, gpu), **kw)
+        assert torch.equal(got[1], ref[1]) and torch.equal(got[0], ref[0])
+
+
 @pytest.mark.parametrize("scale", [1e-6, 1.0, 1e6])
 def test_clusters_of_very_different_density(gpu, scale):
     """Clusters a thousandth of the scene wide beside sparse sites (a Morton

@@ -69,13 +69,52 @@ constexpr int NV_SMALL = 1, NV_MID = 2, NV_LARGE = 8;
 // the first with at most 64.
 constexpr uint32_t VOR_LEAF = 8;
 constexpr int VOR_LEVELS = 4; // 8 * 64^4 sites and more: 2^27
+struct VorBox;
 struct VorTree {
     const float4 *sites;               // sorted (x, y, z, original index)
     const float4 *boxes;               // (lo, -), (hi, -) per box, level after level
     uint32_t count[VOR_LEVELS];
     int top;
-    const float *bbox;                 // of all sites (6 floats)
+    const VorBox *box;
 };
+
+// The builder works on the sites scaled by 2^-k, k the exponent of their
+// largest extent (exact, and Voronoi neighbours do not depend on scale): the
+// f32 squares and lengths that rule sites out then neither overflow nor
+// underflow, whatever unit the sites are in.  Unscaled squares left the builder
+// with wrong lists from extents of 2^44 on and at 2^-70.
+struct VorBox {
+    double lo[3], hi[3]; // what every cell starts as (scaled)
+    double diag2;        // squared diagonal of the sites' own box
+    int k;
+};
+
+// No scale for one place or sites that are not finite.  Extents below 1e-6
+// count as 1e-6, down to 2^-40 of that.
+__device__ __forceinline__ void scaled_box(const float *bbox, VorBox &b)
+{
+    double ext = 0.0;
+    for (int a = 0; a < 3; ++a)
+        ext = fmax(ext, (double)bbox[3 + a] - (double)bbox[a]);
+    b.k = ext > 0.0 && ext < 1e39 ? min(max(ilogb(ext), -126), 126) : 0;
+    double most = fmin(ldexp(1e-6, -b.k), 0x1p40);
+    b.diag2 = 0.0;
+    for (int a = 0; a < 3; ++a) {
+        b.lo[a] = ldexp((double)bbox[a], -b.k);
+        b.hi[a] = ldexp((double)bbox[3 + a], -b.k);
+        b.diag2 = fma(b.hi[a] - b.lo[a], b.hi[a] - b.lo[a], b.diag2);
+        most = fmax(most, b.hi[a] - b.lo[a]);
+    }
+    for (int a = 0; a < 3; ++a) {
+        b.lo[a] -= 1e6 * most;
+        b.hi[a] += 1e6 * most;
+    }
+}
+__device__ __forceinline__ float4 scaled_site(const float *points, uint32_t i, int k)
+{
+    const float *p = points + 3 * (size_t)i;
+    return make_float4(ldexpf(p[0], -k), ldexpf(p[1], -k), ldexpf(p[2], -k), __uint_as_float(i));
+}
 
 // Boxes before a level's first (level wave-uniform: scalar selects).
 __host__ __device__ __forceinline__ uint32_t level_begin(const VorTree &t, int level)
@@ -785,21 +824,14 @@ __device__ __forceinline__ int offer_tree(VorLds<NV> &s, VorCell<NV> &c, const V
 // edge of the closed triangulation appears once in each direction.  Across
 // the edge of two planes lies the corner on the other plane of the third axis.
 template <int NV>
-__device__ __forceinline__ double cell_begin(VorLds<NV> &s, VorCell<NV> &c, const VorTree &t, const VorReach &r, int lane)
+__device__ __forceinline__ void cell_begin(VorLds<NV> &s, VorCell<NV> &c, const VorTree &t, const VorReach &r, int lane)
 {
     const double p[3] = {(double)r.px, (double)r.py, (double)r.pz};
-    double lo[3], hi[3], most = 0.0, diag2 = 0.0;
+    double lo[3], hi[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        lo[a] = (double)t.bbox[a];
-        hi[a] = (double)t.bbox[3 + a];
-        diag2 = fma(hi[a] - lo[a], hi[a] - lo[a], diag2);
-        most = fmax(most, fmax(hi[a] - lo[a], 1e-6));
-    }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        lo[a] = lo[a] - 1e6 * most - p[a];
-        hi[a] = hi[a] + 1e6 * most - p[a];
+        lo[a] = t.box->lo[a] - p[a];
+        hi[a] = t.box->hi[a] - p[a];
     }
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
@@ -832,7 +864,6 @@ __device__ __forceinline__ double cell_begin(VorLds<NV> &s, VorCell<NV> &c, cons
     }
     c.full = 0;
     lds_sync();
-    return diag2;
 }
 
 // Sites on common spheres leave faces of no area, which planes offered in one
@@ -921,7 +952,8 @@ __device__ __forceinline__ int voronoi_cell(VorLds<NV> &s, VorCell<NV> &c, const
     const uint32_t self = __float_as_uint(own.w);
     VorReach r{own.x, own.y, own.z, 0.0f, 0.0f};
     *m_out = 0;
-    const float diag2 = (float)cell_begin(s, c, t, r, lane); // no two sites are farther apart
+    cell_begin(s, c, t, r, lane);
+    const float diag2 = (float)t.box->diag2; // no two sites are farther apart
     // seeds, one per lane: the guesses, or the 64 sites around it on the curve
     uint32_t first = at < 32u ? 0u : at - 32u;
     if (first + 64u > n)
@@ -941,8 +973,7 @@ __device__ __forceinline__ int voronoi_cell(VorLds<NV> &s, VorCell<NV> &c, const
             site = gadj[gb + lane];
             ok = site < n && site != self;
             if (ok)
-                p = make_float4(points[3 * (size_t)site], points[3 * (size_t)site + 1], points[3 * (size_t)site + 2],
-                                0.0f);
+                p = scaled_site(points, site, t.box->k);
         }
     } else if (first + (uint32_t)lane < n) {
         p = t.sites[first + lane];
@@ -1138,18 +1169,24 @@ __device__ __forceinline__ uint32_t spread10(uint32_t x)
 // Morton codes on a cubic grid of 2^20 steps per axis over the largest
 // extent: the upper 10 bits of each axis in hi, the lower 10 in lo.
 __global__ void voronoi_keys_kernel(const float *__restrict__ points, uint32_t n, const float *__restrict__ bbox,
-                                    uint32_t *__restrict__ hi, uint32_t *__restrict__ lo, uint32_t *__restrict__ vals)
+                                    const VorBox *__restrict__ box, uint32_t *__restrict__ hi,
+                                    uint32_t *__restrict__ lo, uint32_t *__restrict__ vals)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
         return;
-    float ext = 1e-30f;
-    for (int a = 0; a < 3; ++a)
-        ext = fmaxf(ext, bbox[3 + a] - bbox[a]);
+    const int k = box->k;
+    const float4 p = scaled_site(points, i, k);
+    float ext = 1e-30f, at[3] = {p.x, p.y, p.z};
+    for (int a = 0; a < 3; ++a) {
+        const float lo = ldexpf(bbox[a], -k);
+        ext = fmaxf(ext, ldexpf(bbox[3 + a], -k) - lo);
+        at[a] -= lo;
+    }
     uint32_t h = 0, l = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const float x = (points[3 * (size_t)i + a] - bbox[a]) / ext * 1048575.0f;
+        const float x = at[a] / ext * 1048575.0f;
         const uint32_t q = (uint32_t)fminf(fmaxf(x, 0.0f), 1048575.0f);
         h |= spread10(q >> 10) << (2 - a);
         l |= spread10(q & 1023u) << (2 - a);
@@ -1172,15 +1209,14 @@ __global__ void voronoi_take_kernel(const uint32_t *__restrict__ src, const uint
 // Sorted sites and the leaf boxes (a box per VOR_LEAF lanes).
 __global__ __launch_bounds__(256) void voronoi_sites_kernel(const float *__restrict__ points,
                                                             const uint32_t *__restrict__ vals, uint32_t n,
+                                                            const VorBox *__restrict__ box,
                                                             float4 *__restrict__ sites, float4 *__restrict__ boxes)
 {
     const uint32_t k = blockIdx.x * 256u + threadIdx.x;
     const float inf = __builtin_huge_valf();
     float lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
     if (k < n) {
-        const uint32_t i = vals[k];
-        const float4 p = make_float4(points[3 * (size_t)i], points[3 * (size_t)i + 1], points[3 * (size_t)i + 2],
-                                     __uint_as_float(i));
+        const float4 p = scaled_site(points, vals[k], box->k);
         sites[k] = p;
         lo[0] = hi[0] = p.x;
         lo[1] = hi[1] = p.y;
@@ -1239,8 +1275,10 @@ __global__ void voronoi_copy_kernel(uint32_t n, const uint32_t *__restrict__ off
         adjacency[b + k] = src[k];
 }
 
-__global__ void voronoi_begin_kernel(uint32_t *fails, uint32_t *last_count)
+__global__ void voronoi_begin_kernel(uint32_t *fails, uint32_t *last_count, const float *bbox, VorBox *box)
 {
+    if (threadIdx.x == F_WORDS + 1)
+        scaled_box(bbox, *box);
     if (threadIdx.x < F_WORDS)
         fails[threadIdx.x] = threadIdx.x == F_FIRST_BAD ? VOR_NONE : 0u;
     if (threadIdx.x == F_WORDS)
@@ -1252,6 +1290,7 @@ struct VorWs {
     uint32_t *lists, *counts, *keys, *keys_lo, *vals, *sort_ws, *scan_ws, *fails, *bbox_ws, *retry[RETRIES], *big_lists,
         *big_slot, *sites, *boxes;
     float *bbox;
+    VorBox *box;
     uint32_t count[VOR_LEVELS];
 };
 
@@ -1283,6 +1322,8 @@ static size_t ws_words(uint32_t n, VorWs *w, uint32_t *base)
     uint32_t *bb;
     take(&bb, 6);
     x.bbox = reinterpret_cast<float *>(bb);
+    take(&bb, sizeof(VorBox) / 4); // (each of these starts at a multiple of 256 bytes)
+    x.box = reinterpret_cast<VorBox *>(bb);
     for (int q = 0; q < RETRIES; ++q)
         take(&x.retry[q], n);
     take(&x.big_lists, (size_t)big_cap_for(n) * BIG_K);
@@ -1331,13 +1372,13 @@ extern "C" int vt_voronoi_build_warm(const float *points, uint32_t num_points, c
     if (rc)
         return rc;
     // sites along a Morton curve, and the boxes over them
-    voronoi_begin_kernel<<<1, 64, 0, s>>>(w.fails, w.counts + n);
+    voronoi_begin_kernel<<<1, 64, 0, s>>>(w.fails, w.counts + n, w.bbox, w.box);
     VT_LAUNCH_CHECK("voronoi_begin_kernel");
     const uint32_t nblocks = (n + 255) / 256;
     const bool fine = n >= FINE_KEYS_MIN;
     uint32_t *lo = w.keys_lo + n;
-    voronoi_keys_kernel<<<nblocks, 256, 0, s>>>(points, n, w.bbox, fine ? w.keys_lo : w.keys, fine ? w.keys : nullptr,
-                                                w.vals);
+    voronoi_keys_kernel<<<nblocks, 256, 0, s>>>(points, n, w.bbox, w.box, fine ? w.keys_lo : w.keys,
+                                                fine ? w.keys : nullptr, w.vals);
     VT_LAUNCH_CHECK("voronoi_keys_kernel");
     rc = radix_sort_pairs(w.keys, w.vals, n, 30, w.sort_ws, s);
     if (rc)
@@ -1351,10 +1392,11 @@ extern "C" int vt_voronoi_build_warm(const float *points, uint32_t num_points, c
     }
     VorTree t{};
     t.sites = reinterpret_cast<const float4 *>(w.sites);
-    t.bbox = w.bbox;
+    t.box = w.box;
     float4 *boxes = reinterpret_cast<float4 *>(w.boxes);
     t.boxes = boxes;
-    voronoi_sites_kernel<<<nblocks, 256, 0, s>>>(points, w.vals, n, reinterpret_cast<float4 *>(w.sites), boxes);
+    voronoi_sites_kernel<<<nblocks, 256, 0, s>>>(points, w.vals, n, w.box, reinterpret_cast<float4 *>(w.sites),
+                                                 boxes);
     VT_LAUNCH_CHECK("voronoi_sites_kernel");
     std::copy(w.count, w.count + VOR_LEVELS, t.count);
     for (t.top = 0; t.top == 0 || w.count[t.top] > 64;) {
