@@ -160,6 +160,29 @@ def test_any_unit(gpu, e):
         assert torch.equal(got[1], ref[1]) and torch.equal(got[0], ref[0])
 
 
+@pytest.mark.parametrize("n", [9, 200, 6000])
+def test_coplanar_sites_on_a_tilted_plane(gpu, n):
+    """Exactly coplanar sites (z = x / 2 + y / 4 on a dyadic grid): every cell is
+    an open column, whose neighbours are those of the plane's own Delaunay
+    triangulation; with a volume of sites above, of the whole set's."""
+    from scipy.spatial import Delaunay
+
+    rng = np.random.default_rng(n)
+    xy = np.unique(np.round(rng.uniform(-1, 1, size=(n, 2)) * 2 ** 16) / 2 ** 16, axis=0)
+    pts = np.concatenate([xy, 0.5 * xy[:, :1] + 0.25 * xy[:, 1:]], axis=1)
+    e = np.array([1.0, 0.0, 0.5]) / np.sqrt(1.25)
+    f = np.array([0.0, 1.0, 0.25]) - 0.1 * np.array([1.0, 0.0, 0.5])
+    flat = np.stack([pts @ e, pts @ f / np.linalg.norm(f)], axis=1)
+    ptr, idx = Delaunay(flat).vertex_neighbor_vertices
+    adj, off, _ = ops.build_voronoi_adjacency(H.to_dev(pts.astype(np.float32), gpu))
+    adj, off = adj.cpu().numpy(), off.cpu().numpy()
+    for i in range(len(pts)):
+        assert np.array_equal(adj[off[i]:off[i + 1]], np.sort(idx[ptr[i]:ptr[i + 1]])), i
+    up = rng.uniform(-1, 1, size=(n, 3))
+    up[:, 2] = 0.5 * up[:, 0] + 0.25 * up[:, 1] + 0.02 + 2 * np.abs(up[:, 2])
+    _check(np.concatenate([pts, up]).astype(np.float32), gpu)
+
+
 @pytest.mark.parametrize("scale", [1e-6, 1.0, 1e6])
 def test_clusters_of_very_different_density(gpu, scale):
     """Clusters a thousandth of the scene wide beside sparse sites (a Morton

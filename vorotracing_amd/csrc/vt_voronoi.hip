@@ -685,8 +685,9 @@ __device__ __forceinline__ uint64_t boxes_in_reach(const VorTree &t, const VorCe
     return __ballot(in && may);
 }
 
-// From this many sites of a batch on, a cell of several vertices per lane tests
-// them all against its vertices one by one instead of offering each.
+// From this many sites of a batch on, they are tested together, one per lane,
+// against one vertex after another (one vertex per lane: the far ones, several:
+// all of them) instead of offering each.
 constexpr int MANY = 8;
 
 // Sites of the leaf boxes s.hits[first, first + 8), one per lane: those that
@@ -729,7 +730,29 @@ __device__ __forceinline__ int offer_sites(VorLds<NV> &s, VorCell<NV> &c, const 
         }
     }
     const VorOffer mine{fx, fy, fz, SLACK * sqrtf(d2f), w};
-    uint64_t m = __ballot(cand && (far_cut || !(sb * (1.0f + SLACK) < w)));
+    const bool near_cut = !(sb * (1.0f + SLACK) < w);
+    if (NV == NV_SMALL && __popcll(__ballot(cand && far_cut && !near_cut)) >= MANY) {
+        // SLACK of a vertex 10^6 extents away passes every site within 10^-5 rad
+        // of its tangent plane: all of them, where sites on a plane leave the
+        // cell open.  cell_cut's own test then, one site per lane (coplanar
+        // sites on a tilted plane, 50,000: 198 -> 36 ms, 100,000: 806 -> 135).
+        // For every batch it cost the 1M heightfield build 5 %, in the larger
+        // passes 2 % where a noisy plane lies below a volume.
+        const double x = (double)p.x - (double)r.px, y = (double)p.y - (double)r.py, z = (double)p.z - (double)r.pz;
+        const double wd = 0.5 * fma(x, x, fma(y, y, z * z));
+        far_cut = false;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            uint64_t a = c.farv[k];
+            while (a) {
+                const int v = (int)__builtin_ctzll(a);
+                a &= a - 1;
+                const double vx = readlane_d(c.v[k].x, v), vy = readlane_d(c.v[k].y, v), vz = readlane_d(c.v[k].z, v);
+                far_cut = far_cut || fma(x, vx, fma(y, vy, z * vz)) > wd;
+            }
+        }
+    }
+    uint64_t m = __ballot(cand && (far_cut || near_cut));
     if (NV > 1 && __popcll(m) >= MANY) {
         // (a cell of many faces: the box of its vertices lets too many pass)
         float most = 0.0f;
