@@ -338,8 +338,10 @@ int vt_trace_infer_q8_camera(const float *points, const uint8_t *diffuse, const 
  *   the first tile_order[tiles] as two half-waves each (rows 0-3, rows 4-7);
  *   a split tile's cost is then the larger of its halves' costs (each
  *   half's longest walk and most face records), recorded with an atomic max:
- *   clear tile_cost before such a call.  With a split count of 0 the order
- *   is ignored (screen order).
+ *   clear tile_cost before such a call.  Launches that run four lanes per
+ *   ray (no stats, at most 1,792 tiles, not half contributions) take the
+ *   order but split nothing.  With a split count of 0 the order is ignored
+ *   (screen order; its other words need not be set).
  */
 int vt_trace_fwd(int attr_dtype, const float *points, const void *diffuse, const void *specular, uint32_t diff_res,
                  uint32_t spec_res, const float *density, const uint32_t *adjacency, uint32_t adjacency_size,
@@ -376,9 +378,10 @@ int vt_trace_fwd(int attr_dtype, const float *points, const void *diffuse, const
  *   are combined in LDS before the global atomics.
  *   tile_order (an extension, ABI version 10): with image lanes or a
  *   ray_perm (tiles as for vt_trace_fwd), NULL or the tiles + 1 words of
- *   vt_tile_order over the costs the forward of these rays recorded.  Tiles launch in that order, and the first
- *   tile_order[tiles] of them (at most vt_train_bwd_resident_waves()) run as
- *   two half-waves of 32 rays each.
+ *   vt_tile_order over the costs the forward of these rays recorded.  Tiles
+ *   launch in that order, and the first tile_order[tiles] of them (at most
+ *   vt_train_bwd_resident_waves()) run as two half-waves of 32 rays each
+ *   (launches with four lanes per ray split nothing).
  */
 int vt_trace_bwd(int attr_dtype, const float *points, const void *diffuse, const void *specular, uint32_t diff_res,
                  uint32_t spec_res, const float *density, const uint32_t *adjacency, uint32_t adjacency_size,

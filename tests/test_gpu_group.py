@@ -121,3 +121,34 @@ def test_contribution_and_point_error(gpu):
     for a, b in zip(sums[0], sums[1]):
         assert float((times * a - b).norm()) <= 1e-5 * float(b.norm())
         assert float(a.sum()) > 0
+
+
+@pytest.mark.parametrize("h,w", [(64, 72), (9, 8)])
+def test_forward_ignores_an_order_without_splits(gpu, monkeypatch, h, w):
+    """vt_trace_fwd: "with a split count of 0 the order is ignored"; its other
+    words are then unset memory, here past the last tile."""
+    m = VoroTracing.from_scene(scene.random_scene(600, seed=9, R=4), device=gpu)
+    scn = (m.primal_points.detach(), m.att_diffuse.detach(), m.att_specular.detach(),
+           m.activated_density().detach(), m.point_adjacency, m.point_adjacency_offsets)
+    rays = _images(gpu, 1, h, w)[0].contiguous()
+    start = m.get_starting_point(rays)
+    tiles = _tiles(rays)
+    order = torch.full((tiles + 1,), 0x7fffffff, dtype=torch.int32, device=gpu)
+    order[tiles] = 0
+    cost = torch.zeros(tiles, dtype=torch.int32, device=gpu)
+
+    class Unset:
+        def __init__(self, o):
+            self.o = o
+
+        def launch_args(self, *args, **kw):
+            cost.zero_()
+            return self.o, cost.data_ptr()
+
+    got = []
+    for o in (None, order.data_ptr()):
+        monkeypatch.setattr(_C, "_train_schedule", lambda *args, o=o: (Unset(o), None))
+        out = _C.trace_vorotracing_fwd(*scn, rays, start, None, 0.001, 1024, False)
+        got.append([x.view(torch.int32).clone() for x in out if x is not None] + [cost.clone()])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    assert int(cost.min()) > 0

@@ -445,11 +445,16 @@ void fwd_kernel(FwdArgs a)
 }
 
 // The block's ray of a group launch (group_within), in the tile that its
-// place in the launch order has (tile NONE: past the last).
+// place in the launch order has.  As in train_slot, the forward
+// (ORDER_ONLY_TO_SPLIT) ignores an order whose split count is 0, whose entries
+// need not even be set; nothing is split here.
+template <bool ORDER_ONLY_TO_SPLIT>
 __device__ __forceinline__ uint32_t group_ray(uint32_t num_rays, const uint32_t *perm, uint32_t ni, uint32_t h,
                                               uint32_t w, const uint32_t *tile_order, uint32_t &tile)
 {
-    tile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
+    tile = blockIdx.x;
+    if (tile_order && (!ORDER_ONLY_TO_SPLIT || tile_order[gridDim.x]))
+        tile = tile_order[tile];
     const bool tiled = ni && !perm;
     const uint32_t q = tile * 64u + group_within(tiled);
     if (tiled)
@@ -467,7 +472,7 @@ __global__ __launch_bounds__(GROUP_BLOCK) void fwd_group_kernel(FwdArgs a)
 {
     __shared__ uint32_t most[2][GROUP_BLOCK / 64];
     uint32_t tile, n = 0, faces = 0;
-    const uint32_t r = group_ray(a.num_rays, a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order, tile);
+    const uint32_t r = group_ray<true>(a.num_rays, a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order, tile);
     if (r != NONE)
         n = fwd_ray<A, RD, RS, false, GROUP>(a, r, faces);
     if (a.tile_cost && (a.num_images || a.ray_perm)) {
@@ -1078,7 +1083,7 @@ __global__ __launch_bounds__(GROUP_BLOCK) void bwd_group_kernel(BwdArgs a)
     __shared__ __align__(16) float rows_lds[GROUP_BLOCK / 64][ROW_TABLE_FLOATS];
     float *rows = begin_rows(rows_lds[threadIdx.x / 64]);
     uint32_t tile;
-    const uint32_t r = group_ray(a.num_rays, a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order, tile);
+    const uint32_t r = group_ray<false>(a.num_rays, a.ray_perm, a.num_images, a.img_h, a.img_w, a.tile_order, tile);
     if (r != NONE)
         bwd_ray<A, RD, RS, false, GROUP, GA>(a, r, rows);
 }
