@@ -373,7 +373,10 @@ int vt_trace_fwd(int attr_dtype, const float *points, const void *diffuse, const
  *   + 3 diff_res^2 + 3 spec_res^2) floats, 16-byte aligned, any contents (an
  *   extension, ABI version 4): the call accumulates each cell's point and
  *   density gradients there, in one 16-byte slot per cell, and adds the
- *   slots into points_grad and density_grad at its end.
+ *   slots into points_grad and density_grad at its end; for
+ *   VT_ATTR_F16_SUMS it sums the texture gradients behind the slots, marks
+ *   the cells that have any in diffuse_grad (each row's first half), and
+ *   rounds those into diffuse_grad and specular_grad.
  *   Gradient scatters of lanes that integrate the same cell in the same step
  *   are combined in LDS before the global atomics.
  *   tile_order (an extension, ABI version 10): with image lanes or a

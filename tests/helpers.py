@@ -236,6 +236,22 @@ def assert_f16_sum_close(got, want, abs_sum, count, name=""):
     assert not g[none].any() and not w[none].any(), f"{name}: a value where nothing was added"
 
 
+def assert_one_rounding(got, sums, abs_sum, count, name=""):
+    """Every half within one rounding of its f32 sum: of ``sums`` (the oracle's,
+    of the same ``count`` terms of absolute sum ``abs_sum``), u |sum| + s, plus
+    what two orders of k f32 terms differ by, 2 k 2^-24 A (twice, as that may
+    move the sum over a rounding boundary)."""
+    g, f = np.asarray(got, np.float32).astype(np.float64), np.asarray(sums, np.float64)
+    assert g.shape == f.shape and np.isfinite(g).all(), name
+    order = 2.0 * np.asarray(count, np.float64) * 2.0 ** -24 * np.asarray(abs_sum, np.float64)
+    allow = F16_U * (np.abs(f) + order) + F16_SUB + order
+    bad = np.nonzero(np.abs(g - f) > allow)
+    assert bad[0].size == 0, (f"{name}: {bad[0].size} elements more than a rounding from their f32 sums, first (got, "
+                              f"sum, allowed) {list(zip(g[bad][:4], f[bad][:4], allow[bad][:4]))}")
+    none = np.asarray(count) == 0
+    assert not g[none].any(), f"{name}: a value where nothing was added"
+
+
 def f16_train_sums(s, rays, start, thr, fw16, g16, contribution=False, **bwd_kw):
     """Absolute sums and add counts (oracle sum modes) of the f16-storage
     training call whose forward outputs are ``fw16`` and upstream gradient

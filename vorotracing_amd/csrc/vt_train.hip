@@ -515,6 +515,7 @@ struct BwdArgs {
     uint32_t max_steps;
     float *cell_grad; // (num_points, 4): point gradient, density gradient
     void *diffuse_grad, *specular_grad;
+    uint16_t *touched; // (VT_ATTR_F16_SUMS) the half diffuse gradients
     void *point_error;
     uint32_t *stats;
     const uint32_t *tile_order; // tiled lane order: launch order of the tiles, or null (screen order)
@@ -550,6 +551,7 @@ template <typename A, int RD, int RS, int G = 1, typename GA = A> struct BwdInte
     const float *qthr, *depth_grad;
     float *cell_grad; // per cell (point gradient x, y, z, density gradient)
     GA *diffuse_grad, *specular_grad;
+    uint16_t *touched; // (VT_ATTR_F16_SUMS) the half diffuse gradients: a cell's first one marks it as having sums
     A *point_error;
     f3 prev_geom, prev_grad, cur_grad, next_grad;
     uint32_t prev_idx;
@@ -624,12 +626,20 @@ template <typename A, int RD, int RS, int G = 1, typename GA = A> struct BwdInte
         return c;
     }
 
+    // (f32 sums of half gradients) a texture column was added for the cell
+    __device__ __forceinline__ void mark(const Column &c, uint32_t cell) const
+    {
+        if (!std::is_same<A, GA>::value && c.k < 24u)
+            touched[(size_t)cell * ND] = 1;
+    }
+
     // One add of a combined column: one atomic instruction for every target
     // (f32), or one per storage type (f16 attributes, f32 slots).
     __device__ __forceinline__ void column_send(const Column &c, uint32_t cell, uint32_t tap, float x)
     {
         if (c.on && tap < c.taps) {
             const size_t i = (size_t)cell * c.stride + 3u * tap + c.off;
+            mark(c, cell);
             if (std::is_same<A, float>::value || !c.attr) {
                 atomicAdd(static_cast<float *>(c.base) + i, x);
             } else {
@@ -662,6 +672,8 @@ template <typename A, int RD, int RS, int G = 1, typename GA = A> struct BwdInte
             if (send)
                 atomicAdd(static_cast<float *>(c.base) + i, x);
         } else if constexpr (std::is_same<GA, float>::value) {
+            if (send)
+                mark(c, cell);
             if (send && !c.attr)
                 atomicAdd(static_cast<float *>(c.base) + i, x);
             else if (send) // point_error
@@ -1025,6 +1037,7 @@ __device__ __forceinline__ void bwd_ray(const BwdArgs &a, uint32_t r, float *row
     it.cell_grad = a.cell_grad;
     it.diffuse_grad = (GA *)a.diffuse_grad;
     it.specular_grad = (GA *)a.specular_grad;
+    it.touched = a.touched;
     it.point_error = (A *)a.point_error;
     it.prev_geom = it.prev_grad = it.cur_grad = it.next_grad = mk(0.0f, 0.0f, 0.0f);
     it.prev_idx = NONE;
@@ -1301,20 +1314,48 @@ __global__ void cell_grad_out_kernel(const float4 *g, float *points_grad, float 
     }
 }
 
-// Half gradients from their f32 sums: one rounding each (the outputs are
-// zero-initialised by the caller, as for the atomics).
-__global__ void attr_sums_clear_kernel(float *sums, size_t n)
+// Half gradients from their f32 sums, one rounding each.  The sums of all
+// cells are cleared, 4 bytes a texel; those of cells without any are not read
+// back, and their gradients stay the zeros that the caller put there: the
+// traversal marks a cell by its first diffuse half (not zero), which the
+// conversion then overwrites.  Grids are bounded and loop: a thread per texel
+// is past HIP's 2^32 threads from 11.2M sites of 8x8 maps on.
+constexpr uint32_t SUMS_BLOCKS = 8192;
+__global__ __launch_bounds__(256) void attr_sums_clear_kernel(float4 *sums, size_t n4)
 {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        sums[i] = 0.0f;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256)
+        sums[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
-__global__ void attr_sums_out_kernel(const float *sums, uint16_t *grad, size_t n)
+// A wave reads the marks of 64 cells and converts the marked ones four at a
+// time, 16 lanes each.
+__global__ __launch_bounds__(256) void attr_sums_out_kernel(const float *dsums, const float *ssums, uint16_t *dgrad,
+                                                            uint16_t *sgrad, uint32_t nd, uint32_t ns,
+                                                            uint32_t num_points)
 {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        grad[i] = f2h(h2f(grad[i]) + sums[i]);
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t waves = (uint64_t)gridDim.x * 4;
+    for (uint64_t c0 = ((uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 64; c0 < num_points; c0 += waves * 64) {
+        const size_t cell = c0 + lane;
+        uint64_t marked = __ballot(cell < num_points && dgrad[cell * nd] != 0);
+        while (marked) {
+            uint64_t mine = marked;
+#pragma unroll
+            for (uint32_t g = 0; g < 4; ++g) {
+                mine = g < lane / 16 ? mine & (mine - 1) : mine;
+                marked &= marked - 1;
+            }
+            if (!mine)
+                continue;
+            const size_t at = c0 + __builtin_ctzll(mine);
+#pragma unroll 4
+            for (uint32_t k = lane % 16; k < nd; k += 16)
+                dgrad[at * nd + k] = f2h(dsums[at * nd + k]);
+#pragma unroll 4
+            for (uint32_t k = lane % 16; k < ns; k += 16)
+                sgrad[at * ns + k] = f2h(ssums[at * ns + k]);
+        }
+    }
 }
 
 extern "C" int vt_trace_bwd(int attr_dtype, const float *points, const void *diffuse, const void *specular,
@@ -1339,7 +1380,8 @@ extern "C" int vt_trace_bwd(int attr_dtype, const float *points, const void *dif
     VT_REQUIRE(num_rays == 0 || (rays && start_point && rgba && rgba_grad), "null ray pointer");
     VT_REQUIRE(points_grad && diffuse_grad && specular_grad && density_grad, "null gradient output");
     VT_REQUIRE(cell_workspace && reinterpret_cast<uintptr_t>(cell_workspace) % 16 == 0,
-               "cell_workspace must be a 16-byte aligned (num_points, 4) float array");
+               "cell_workspace must be 16-byte aligned: num_points * 4 floats, with f32 sums of half gradients 4 and one "
+               "per texel value");
     VT_REQUIRE(!depth_quantiles || num_quantiles == 0 || (depth_idx && depth_grad),
                "depth_idx and depth_grad required when depth_quantiles is given");
     VT_REQUIRE(!ray_error || point_error, "point_error output required when ray_error is given");
@@ -1388,18 +1430,21 @@ extern "C" int vt_trace_bwd(int attr_dtype, const float *points, const void *dif
     const uint32_t cblocks = (num_points + 255) / 256;
     cell_grad_clear_kernel<<<cblocks, 256, 0, s>>>(reinterpret_cast<float4 *>(cell_workspace), num_points);
     VT_LAUNCH_CHECK("cell_grad_clear_kernel");
-    const size_t nd = (size_t)num_points * 3 * diff_res * diff_res, ns = (size_t)num_points * 3 * spec_res * spec_res;
     if (attr_dtype == VT_ATTR_F16_SUMS) {
-        float *attr_sums = cell_workspace + 4 * (size_t)num_points;
-        a.diffuse_grad = attr_sums;
-        a.specular_grad = attr_sums + nd;
-        attr_sums_clear_kernel<<<(uint32_t)((nd + ns + 255) / 256), 256, 0, s>>>(attr_sums, nd + ns);
+        const uint32_t nd = 3 * diff_res * diff_res, ns = 3 * spec_res * spec_res; // multiples of 4 (checked maps)
+        float *dsums = cell_workspace + 4 * (size_t)num_points, *ssums = dsums + (size_t)num_points * nd;
+        a.diffuse_grad = dsums;
+        a.specular_grad = ssums;
+        a.touched = (uint16_t *)diffuse_grad;
+        const size_t n4 = (size_t)num_points * ((nd + ns) / 4);
+        attr_sums_clear_kernel<<<(uint32_t)std::min<size_t>((n4 + 255) / 256, SUMS_BLOCKS), 256, 0, s>>>(
+            reinterpret_cast<float4 *>(dsums), n4);
         VT_LAUNCH_CHECK("attr_sums_clear_kernel");
         rc = launch_train_a<BwdSumsK, BwdArgs, uint16_t>(a, diff_res, spec_res, stats != nullptr, s);
         if (rc)
             return rc;
-        attr_sums_out_kernel<<<(uint32_t)((nd + 255) / 256), 256, 0, s>>>(attr_sums, (uint16_t *)diffuse_grad, nd);
-        attr_sums_out_kernel<<<(uint32_t)((ns + 255) / 256), 256, 0, s>>>(attr_sums + nd, (uint16_t *)specular_grad, ns);
+        attr_sums_out_kernel<<<std::min((num_points + 255) / 256, SUMS_BLOCKS), 256, 0, s>>>(
+            dsums, ssums, (uint16_t *)diffuse_grad, (uint16_t *)specular_grad, nd, ns, num_points);
         VT_LAUNCH_CHECK("attr_sums_out_kernel");
     } else {
         rc = launch_train<BwdK>(attr_dtype, a, diff_res, spec_res, stats != nullptr, s);
