@@ -75,9 +75,44 @@ def test_half_gradients_are_rounded_once(gpu, which, error):
             A["point_error"], K["point_error"], "point_error")
 
 
-def test_more_texels_than_a_grid_has_threads(gpu):
+@pytest.mark.parametrize("why", ["size", "memory"])
+@pytest.mark.parametrize("which,error", [("image", False), ("image", True), ("87", False), ("7", False)])
+def test_half_atomics(gpu, monkeypatch, why, which, error):
+    """Past the sizes up to which the sums pay, and where they cannot be
+    allocated, gradients are added with half atomics (VT_ATTR_F16): within the
+    accumulation bound of the oracle's half sums."""
+    s, rays = _scene(which)
+    if why == "size":
+        monkeypatch.setattr(_C, "SUMS_VALUES", 0)
+        monkeypatch.setattr(_C, "SUMS_VALUES_PER_RAY", 0)
+    else:
+        empty, slots = torch.empty, 4 * s.points.shape[0]
+
+        def no_memory(*size, **kw):
+            if kw.get("dtype") == torch.float32 and isinstance(size[0], int) and size[0] > slots:
+                raise torch.OutOfMemoryError("no memory for the sums")
+            return empty(*size, **kw)
+
+        monkeypatch.setattr(torch, "empty", no_memory)
+    codes = []
+    workspace = _C._cell_workspace
+    monkeypatch.setattr(_C, "_cell_workspace", lambda *a: codes.append(workspace(*a)) or codes[-1])
+    out, start, fw, g, e = _backward(s, rays, error, gpu)
+    assert [c[0] for c in codes] == [1] and codes[0][1].numel() == 4 * s.points.shape[0]
+    want = core.trace_bwd(s.points, s.diffuse.astype(np.float16), s.specular.astype(np.float16), s.diff_res, s.spec_res,
+                          s.density, s.adjacency, s.offsets, rays, start, fw["rgba"], g, ray_error=e,
+                          distortion=fw["distortion"], W_total=fw["W_total"], S_total=fw["S_total"], t_far=fw["t_far"],
+                          weight_threshold=0.001)
+    _, A, K = _oracle_sums(s, rays, start, fw, g, e)
+    for got, key in ((out[1], "diffuse_grad"), (out[2], "specular_grad")) + (((out[5], "point_error"),) if error else ()):
+        H.assert_f16_sum_close(got.cpu().numpy(), want[key], A[key], K[key], key)
+    H.assert_grad_close(out[0].cpu().numpy(), want["points_grad"], "points_grad", abs_sum=A["points_grad"])
+
+
+def test_more_texels_than_a_grid_has_threads(gpu, monkeypatch):
     """11.3 million cells of 8x8 and 8x8 maps are 4.3e9 texels: more than 2^32,
     which bounds a grid's threads.  The cells that the rays meet are the last."""
+    monkeypatch.setattr(_C, "SUMS_VALUES", 1 << 40)
     s = H.small_random(400, seed=11, R=8, Rs=8)
     rays = camera.pinhole_rays(24, 16, eye=(0.3, -3.2, 0.4))
     pad = 11_300_000

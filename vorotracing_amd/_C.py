@@ -590,6 +590,30 @@ def _stats_ptr(stats: Optional[torch.Tensor], num_rays: int):
     return stats.data_ptr()
 
 
+# Half maps have their gradients summed in f32 and rounded once up to this many
+# texel values, or this many a ray: clearing the sums, 4 bytes a value, costs
+# less there than f32 atomics save against half ones.  Backward of 8x8 maps with
+# half atomics / with sums, ms: 3M sites (1.15e9 values) 1,024 rays 6.5 / 3.4,
+# 262,144 rays 9.0 / 8.8; 8M sites (3.1e9) 65,536 rays 9.2 / 9.3 and with ray_error 9.3 / 11.6, 262,144 rays
+# 16.5 / 17.6, a million rays 40.0 / 37.9.
+SUMS_VALUES = 1_200_000_000
+SUMS_VALUES_PER_RAY = 4096
+
+
+def _cell_workspace(code: int, num_points: int, values: int, num_rays: int, dev):
+    """(attribute code, cell workspace) of a training backward over maps of
+    ``values`` texel values.  Half maps: VT_ATTR_F16_SUMS with the f32 sums
+    behind the cells' slots, or VT_ATTR_F16 (half atomics, a rounding at every
+    add, as the reference) past the sizes above and where the sums, twice the
+    gradients' memory, cannot be allocated."""
+    if code == 1 and values <= max(SUMS_VALUES, SUMS_VALUES_PER_RAY * num_rays):
+        try:
+            return 2, torch.empty(4 * num_points + values, dtype=torch.float32, device=dev)
+        except torch.OutOfMemoryError:
+            pass
+    return code, torch.empty((num_points, 4), dtype=torch.float32, device=dev)
+
+
 def trace_vorotracing_bwd(points_in, diffuse_in, specular_in, density_in, point_adjacency_in,
                           point_adjacency_offsets_in, rays_in, start_point_in, rgb_out, rgb_grad_in,
                           depth_quantiles_in, depth_indices_in, depth_grad_in, ray_error_in,
@@ -681,10 +705,7 @@ def trace_vorotracing_bwd(points_in, diffuse_in, specular_in, density_in, point_
     points_grad = torch.zeros((num_points, 3), dtype=rays.dtype, device=dev)
     ray_grad = torch.zeros_like(rays)
     workspace = _adj_diff_buffer(adj_diff, adjacency_size, dev, "adj_diff")
-    # half maps: their gradients are summed in f32, behind the cells' slots, and rounded once
-    sums = diffuse.numel() + specular.numel() if code == 1 else 0
-    cell_workspace = torch.empty(4 * num_points + sums, dtype=torch.float32, device=dev)
-    code = 2 if code == 1 else code
+    code, cell_workspace = _cell_workspace(code, num_points, diffuse.numel() + specular.numel(), num_rays, dev)
     img_h, img_w, perm = _lane_order(rays, start_point, num_points, ray_perm)
     with torch.cuda.device(dev):
         sch, frame = _train_schedule(rays_in, img_h, img_w, num_rays, perm, ray_perm, dev)
