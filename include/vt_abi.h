@@ -536,8 +536,15 @@ int vt_tile_perm(uint32_t height, uint32_t width, uint32_t tile_h, uint32_t tile
  * vt_train_bwd_resident_waves()), and so does the forward when the count is
  * non-zero (pass vt_train_fwd_resident_waves()); the inference entries
  * ignore the count (pass 0).
+ * split_waves may have VT_TILE_ORDER_LOAD added (at most 2^30 - 1 tiles):
+ * tile_order[tiles] then has bit 31 set when the longest tile costs more than
+ * 1/1228 of sum(cost) and bit 30 when more than 1/1434, the count below them.
+ * The training backward chooses between one and four lanes per ray by these
+ * bits where the number of tiles does not decide (orders without them give
+ * one lane there).
  * workspace: vt_tile_order_workspace_size(tiles) bytes, 8-byte aligned.
  */
+#define VT_TILE_ORDER_LOAD 0x80000000u
 size_t vt_tile_order_workspace_size(uint32_t tiles);
 int vt_tile_order(const uint32_t *tile_cost, uint32_t tiles, uint32_t split_waves, uint32_t *tile_order,
                   void *workspace, vt_stream_t stream);

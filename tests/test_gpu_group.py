@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from tests import helpers as H
-from vorotracing_amd import _C, camera, scene
+from vorotracing_amd import _C, _lib, camera, scene
 from vorotracing_amd.infer import VoroTracingInfer
 from vorotracing_amd.model import VoroTracing
 
@@ -152,3 +152,70 @@ def test_forward_ignores_an_order_without_splits(gpu, monkeypatch, h, w):
         got.append([x.view(torch.int32).clone() for x in out if x is not None] + [cost.clone()])
     assert all(torch.equal(a, b) for a, b in zip(*got))
     assert int(cost.min()) > 0
+
+
+@pytest.mark.parametrize("tiles", [1, 255, 257, 2000])
+@pytest.mark.parametrize("split_waves", [0, 4096])
+def test_order_says_how_even_the_load_is(gpu, tiles, split_waves):
+    """VT_TILE_ORDER_LOAD: bits 31 and 30 of the word after the order, for costs
+    around both limits; order and split count as without it."""
+    ws = torch.empty(int(_lib.load().vt_tile_order_workspace_size(tiles)), dtype=torch.uint8, device=gpu)
+    rng = np.random.default_rng(tiles)
+    for longest in (1000, 1220, 1240, 1420, 1450, 2000):
+        cost = rng.integers(500, 900, size=tiles)
+        # the last tile costs the others' sum over (longest - 1): sum / max = longest, near enough
+        cost[-1] = max(cost[:-1].sum() // (longest - 1), 1) if tiles > 1 else 700
+        total, most = int(cost.sum()), int(cost.max())
+        c = torch.from_numpy(cost.astype(np.int32)).to(gpu)
+        got = []
+        for flag in (0, 1 << 31):
+            order = torch.empty(tiles + 1, dtype=torch.int32, device=gpu)
+            _lib.call("vt_tile_order", c.data_ptr(), tiles, split_waves | flag, order.data_ptr(), ws.data_ptr(),
+                      torch.cuda.current_stream(gpu).cuda_stream)
+            got.append(order.cpu().numpy().view(np.uint32).astype(np.int64))
+        assert np.array_equal(got[0][:tiles], got[1][:tiles])
+        assert got[1][tiles] == got[0][tiles] | (most * 1228 > total) << 31 | (most * 1434 > total) << 30
+
+
+@pytest.mark.parametrize("flat", [False, True])
+@pytest.mark.parametrize("even", [False, True])
+def test_backward_chosen_by_the_load(gpu, even, flat):
+    """Between the lines the costs of the forward choose the kernel that runs:
+    launches as long as their longest tile (four lanes) and launches of tiles
+    all alike (one lane) have the gradients of the launch without an order."""
+    m = VoroTracing.from_scene(scene.random_scene(600, seed=9, R=4), device=gpu)
+    scn = (m.primal_points.detach(), m.att_diffuse.detach(), m.att_specular.detach(),
+           m.activated_density().detach(), m.point_adjacency, m.point_adjacency_offsets)
+    image = _images(gpu, 1, 64, 72)[0]
+    if even:
+        image = image[24:32, 32:40].repeat(8, 9, 1).contiguous()
+    rays = image.repeat(31, 1, 1, 1).contiguous()
+    if not even:
+        rays[8:, ..., 3:] *= -1.0  # away from the scene: a few steps
+    tiles = _tiles(rays)
+    assert 1920 < tiles <= 3072
+    perm = None
+    if flat:  # the lane order that makes the same tiles of 64 rays
+        n = torch.arange(rays.numel() // 6, device=gpu).reshape(31, 8, 8, 9, 8)
+        perm = n.permute(0, 1, 3, 2, 4).reshape(-1).to(torch.int32).contiguous()
+        rays = rays.reshape(-1, 6)
+    start = m.get_starting_point(rays)
+    g = torch.randn(list(rays.shape[:-1]) + [4], generator=torch.Generator(device=gpu).manual_seed(2), device=gpu)
+    got, saved = [], _C.TRAIN_TILE_ORDER
+    try:
+        for order in (False, True):
+            _C.TRAIN_TILE_ORDER = order
+            _C._TRAIN_SCHEDULES.clear()
+            out = _C.trace_vorotracing_fwd(*scn, rays, start, None, 0.001, 1024, False, ray_perm=perm)
+            got.append(_C.trace_vorotracing_bwd(*scn, rays, start, out[0], g, None, None, None, None, 0.0, out[5], None,
+                                                out[6], out[7], out[8], 0.001, 1024, ray_perm=perm)[:4])
+        sch = next(iter(_C._TRAIN_SCHEDULES.values()))
+        word = int(sch.order.view(torch.int32)[tiles].item())
+        cost = sch.cost.view(torch.int32).long()
+    finally:
+        _C.TRAIN_TILE_ORDER = saved
+        _C._TRAIN_SCHEDULES.clear()
+    long = int(cost.max()) * (1434 if flat else 1228) > int(cost.sum())
+    assert long == (not even) and bool(word & (1 << (30 if flat else 31))) == long
+    for a, b in zip(*got):
+        assert float((a.double() - b.double()).norm()) <= 1e-5 * float(a.double().norm()) and float(a.abs().sum()) > 0

@@ -533,7 +533,8 @@ constexpr uint64_t SPLIT_NUM = 4, SPLIT_DEN = 5;
 __global__ __launch_bounds__(TO_BLOCK) void tile_scatter_kernel(const uint32_t *__restrict__ cost, uint32_t tiles,
                                                                 const uint32_t *__restrict__ hist,
                                                                 const uint64_t *__restrict__ total,
-                                                                uint32_t split_waves, uint32_t *__restrict__ order)
+                                                                uint32_t split_waves, bool load,
+                                                                uint32_t *__restrict__ order)
 {
     __shared__ uint32_t base[TO_BINS];
     __shared__ uint32_t wcnt[TO_BLOCK / 64][TO_BINS];
@@ -568,6 +569,11 @@ __global__ __launch_bounds__(TO_BLOCK) void tile_scatter_kernel(const uint32_t *
     const uint64_t tot = *total;
     if (valid && split_waves && tot < (1ull << 57) && SPLIT_DEN * (uint64_t)c * split_waves > SPLIT_NUM * tot)
         atomicAdd(&nsplit, 1u);
+    if (load) { // set by every wave that has such a tile
+        const uint64_t flat = __ballot((uint64_t)c * LOAD_FLAT > tot), image = __ballot((uint64_t)c * LOAD_IMAGE > tot);
+        if (lane == 0 && flat)
+            atomicOr(order + tiles, ORDER_LONG_FLAT | (image ? ORDER_LONG_IMAGE : 0u));
+    }
     __syncthreads();
     if (valid) {
         uint32_t pos = base[key] + rank;
@@ -598,7 +604,10 @@ extern "C" int vt_tile_order(const uint32_t *tile_cost, uint32_t tiles, uint32_t
         return VT_OK;
     VT_REQUIRE(tile_cost && tile_order && workspace, "null pointer argument");
     VT_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 8 == 0, "workspace must be 8-byte aligned");
+    const bool load = split_waves & VT_TILE_ORDER_LOAD;
+    split_waves &= ~VT_TILE_ORDER_LOAD;
     VT_REQUIRE(split_waves < (1u << 24), "split_waves (%u) must be below 2^24", split_waves);
+    VT_REQUIRE(!load || tiles <= ORDER_COUNT, "too many tiles (%u) for VT_TILE_ORDER_LOAD", tiles);
     hipStream_t s = as_stream(stream);
     const uint32_t blocks = tile_order_blocks(tiles);
     uint32_t *hist = static_cast<uint32_t *>(workspace);
@@ -609,7 +618,7 @@ extern "C" int vt_tile_order(const uint32_t *tile_cost, uint32_t tiles, uint32_t
     VT_LAUNCH_CHECK("tile_hist_kernel");
     tile_scan_kernel<<<1, TO_SCAN_THREADS, 0, s>>>(hist, blocks * TO_BINS, psum, blocks, total, tile_order + tiles);
     VT_LAUNCH_CHECK("tile_scan_kernel");
-    tile_scatter_kernel<<<blocks, TO_BLOCK, 0, s>>>(tile_cost, tiles, hist, total, split_waves, tile_order);
+    tile_scatter_kernel<<<blocks, TO_BLOCK, 0, s>>>(tile_cost, tiles, hist, total, split_waves, load, tile_order);
     VT_LAUNCH_CHECK("tile_scatter_kernel");
     return VT_OK;
 }

@@ -189,7 +189,7 @@ __device__ __forceinline__ TrainSlot train_slot(uint32_t s, uint32_t tiles, cons
     }
     const uint32_t waves = gridDim.x * (blockDim.x / 64u);
     const uint32_t extra = waves > tiles ? waves - tiles : 0u;
-    const uint32_t k = min(min(tile_order[tiles], tiles), extra);
+    const uint32_t k = min(min(tile_order[tiles] & ORDER_COUNT, tiles), extra);
     if (ORDER_ONLY_TO_SPLIT && k == 0) {
         if (r.tile >= tiles)
             r.tile = NONE;
@@ -453,7 +453,7 @@ __device__ __forceinline__ uint32_t group_ray(uint32_t num_rays, const uint32_t 
                                               uint32_t w, const uint32_t *tile_order, uint32_t &tile)
 {
     tile = blockIdx.x;
-    if (tile_order && (!ORDER_ONLY_TO_SPLIT || tile_order[gridDim.x]))
+    if (tile_order && (!ORDER_ONLY_TO_SPLIT || tile_order[gridDim.x] & ORDER_COUNT))
         tile = tile_order[tile];
     const bool tiled = ni && !perm;
     const uint32_t q = tile * 64u + group_within(tiled);
@@ -516,6 +516,7 @@ struct BwdArgs {
     float *cell_grad; // (num_points, 4): point gradient, density gradient
     void *diffuse_grad, *specular_grad;
     uint16_t *touched; // (VT_ATTR_F16_SUMS) the half diffuse gradients
+    bool by_load; // both kernels are launched, and the order's load bits choose the one that runs
     void *point_error;
     uint32_t *stats;
     const uint32_t *tile_order; // tiled lane order: launch order of the tiles, or null (screen order)
@@ -1075,10 +1076,20 @@ __device__ __forceinline__ float *begin_rows(float *rows)
     return rows;
 }
 
+// (by_load) Is the launch as long as its longest tile, so that four lanes per
+// ray run it?
+__device__ __forceinline__ bool group_by_load(const BwdArgs &a)
+{
+    const uint32_t tiles = train_tiles(a.num_rays, a.ray_perm != nullptr, a.num_images, a.img_h, a.img_w);
+    return a.tile_order[tiles] & (a.ray_perm ? ORDER_LONG_FLAT : ORDER_LONG_IMAGE);
+}
+
 template <typename A, int RD, int RS, bool STATS, typename GA = A>
 __global__ __launch_bounds__(TRAIN_BLOCK) __attribute__((amdgpu_waves_per_eu(TRAIN_BWD_WAVES)))
 void bwd_kernel(BwdArgs a)
 {
+    if (!STATS && a.by_load && group_by_load(a))
+        return;
     __shared__ __align__(16) float rows_lds[TRAIN_WAVES][ROW_TABLE_FLOATS];
     float *rows = begin_rows(rows_lds[threadIdx.x / 64]);
     const uint32_t r = train_ray<false>(xcd_interleaved_block<TRAIN_XCD_CHUNK>() * blockDim.x + threadIdx.x,
@@ -1093,6 +1104,8 @@ void bwd_kernel(BwdArgs a)
 template <typename A, int RD, int RS, typename GA = A>
 __global__ __launch_bounds__(GROUP_BLOCK) void bwd_group_kernel(BwdArgs a)
 {
+    if (a.by_load && !group_by_load(a))
+        return;
     __shared__ __align__(16) float rows_lds[GROUP_BLOCK / 64][ROW_TABLE_FLOATS];
     float *rows = begin_rows(rows_lds[threadIdx.x / 64]);
     uint32_t tile;
@@ -1133,13 +1146,31 @@ static uint32_t resident_waves(uint32_t waves_per_simd)
 // Launches of up to this many tiles (64 rays each) run with four lanes per ray.
 // One wave per tile leaves the chip's 1,024 SIMDs a wave or two each and lasts
 // as long as its longest wave whatever their number; four waves per tile fill
-// it, and lose once they no longer fit at once.  Torus scene of 131,072 sites,
-// entry times in us with a wave per tile / four:
-//   tiles      1,024        2,025        3,025        4,096
-//   forward    858 / 530    842 / 678    870 / 811    939 / 1,011
-//   backward  2,381 / 1,280  2,459 / 1,520             2,432 / 2,540
-// (heightfield, 2,025 tiles: forward 606 / 615, backward 1,376 / 1,350).
-constexpr uint32_t FWD_GROUP_TILES = 1792, BWD_GROUP_TILES = 3072;
+// it, with more instructions in all.
+// Forward (107 VGPRs, 1,024 blocks resident), the entry's time with four over
+// one, four scenes of 65,536 to 1M sites: 1,024 tiles 0.57 to 0.75, 1,444 0.58
+// to 0.94, 1,764 0.56 to 0.95.
+// Backward in f32 (160 VGPRs, 768 blocks resident): images 1,024 tiles 0.50 to
+// 0.83, 1,536 (two rounds of blocks) 0.69 to 0.90, 1,600 0.73 to 1.03, 2,025
+// 0.60 to 1.10, 3,025 0.81 to 1.04; sorted flat batches 1,407 0.58 to 0.86,
+// 1,922 0.64 to 1.00, 2,344 0.72 to 1.16, 2,813 0.75 to 1.22.
+constexpr uint32_t FWD_GROUP_TILES = 1792, BWD_GROUP_TILES = 1536, BWD_GROUP_WAVES = 1920;
+// Between those lines and this one the scene decides: four lanes win where one
+// lane's launch is as long as its longest tile (a torus or a shell before an
+// empty background, 0.52 to 0.89), and lose where all tiles are alike (a height
+// field that fills the frame, to 1.22).  sum(cost) / max(cost), the number of
+// tiles like the longest that would be as much work, tells: up to 1,228, 1.2
+// per SIMD, images stay below 1 (and reach 1.06 at 1,279); flat batches, whose
+// waves meet more cells, win up to 1,434 by 10 % and more or lose 2 to 4 %
+// there (16 % at 1,501).  The costs are the forward's, on the device, so both
+// kernels are launched and one of them ends at once; without an order over them
+// (another frame came between) one wave runs a tile.  12 scenes, 7 image sizes
+// and 6 flat batches of 1,444 to 3,025 tiles: 0.51 to 1.03 of one lane's time,
+// once 1.05.
+constexpr uint32_t BWD_LOAD_TILES = 3072;
+// Half gradients in f32 sums: four lanes up to this many tiles, 0.35 to 0.97 of
+// the time with half atomics and one lane, 1.02 at 1M sites of 8x8 maps.
+constexpr uint32_t BWD_SUMS_GROUP_TILES = 3072;
 
 template <typename A> constexpr bool F16 = std::is_same<A, uint16_t>::value;
 
@@ -1148,6 +1179,7 @@ template <typename A, int RD, int RS, bool ST> struct FwdK {
     static constexpr auto group_fn = fwd_group_kernel<A, RD, RS>;
     // (a contribution in half storage keeps the wave's larger sums: below)
     static uint32_t group_tiles(const FwdArgs &a) { return F16<A> && a.contribution ? 0u : FWD_GROUP_TILES; }
+    static bool group_by_load(FwdArgs &, uint64_t) { return false; }
     static uint32_t resident() { return resident_waves(TRAIN_FWD_WAVES); }
 };
 template <typename A, int RD, int RS, bool ST> struct BwdK {
@@ -1156,7 +1188,11 @@ template <typename A, int RD, int RS, bool ST> struct BwdK {
     // 16 rays of a wave meet in fewer f32 sums than 64, so half gradients
     // would be rounded more often (their error against 64 bits 0.0028 with a
     // wave per tile, 0.0040 with four)
-    static uint32_t group_tiles(const BwdArgs &) { return F16<A> ? 0u : BWD_GROUP_TILES; }
+    static uint32_t group_tiles(const BwdArgs &a) { return F16<A> ? 0u : a.ray_perm ? BWD_GROUP_WAVES : BWD_GROUP_TILES; }
+    static bool group_by_load(BwdArgs &a, uint64_t tiles)
+    {
+        return a.by_load = !F16<A> && a.tile_order && tiles <= BWD_LOAD_TILES;
+    }
     static uint32_t resident() { return resident_waves(TRAIN_BWD_WAVES); }
 };
 // Half attributes whose texture gradients are summed in f32: f32 atomics in
@@ -1167,20 +1203,23 @@ template <typename A, int RD, int RS, bool ST> struct BwdK {
 template <typename A, int RD, int RS, bool ST> struct BwdSumsK {
     static constexpr auto fn = bwd_kernel<uint16_t, RD, RS, ST, float>;
     static constexpr auto group_fn = bwd_group_kernel<uint16_t, RD, RS, float>;
-    static uint32_t group_tiles(const BwdArgs &a) { return a.point_error ? 0u : BWD_GROUP_TILES; }
+    static uint32_t group_tiles(const BwdArgs &a) { return a.point_error ? 0u : BWD_SUMS_GROUP_TILES; }
+    static bool group_by_load(BwdArgs &, uint64_t) { return false; }
     static uint32_t resident() { return resident_waves(TRAIN_BWD_WAVES); }
 };
 
 template <template <typename, int, int, bool> class K, typename Args, typename A, int RD, int RS>
-static int launch_train_rs(const Args &a, bool stats, hipStream_t s)
+static int launch_train_rs(Args a, bool stats, hipStream_t s)
 {
     using Kernel = K<A, RD, RS, false>;
     const uint64_t all = a.num_images && !a.ray_perm ? train_tiles(a.num_rays, false, a.num_images, a.img_h, a.img_w)
                                                      : ((uint64_t)a.num_rays + 63) / 64;
-    if (!stats && all <= Kernel::group_tiles(a)) {
+    const bool group = !stats && all <= Kernel::group_tiles(a);
+    if (group || (!stats && Kernel::group_by_load(a, all))) {
         hipLaunchKernelGGL((Kernel::group_fn), dim3((uint32_t)all), dim3(GROUP_BLOCK), 0, s, a);
         VT_LAUNCH_CHECK("training traversal kernel (four lanes per ray)");
-        return VT_OK;
+        if (group)
+            return VT_OK;
     }
     uint64_t slots = a.num_rays;
     if (a.num_images || a.ray_perm) {

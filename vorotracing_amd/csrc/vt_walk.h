@@ -654,6 +654,12 @@ __device__ __forceinline__ uint32_t tile_cost_of(uint32_t steps_max, uint32_t fa
     return TILE_COST_STEP * steps_max + faces_max;
 }
 
+// The word after a launch order: the split count and, with VT_TILE_ORDER_LOAD,
+// whether the longest tile costs more than sum(cost) / LOAD_IMAGE, or
+// sum(cost) / LOAD_FLAT (vt_train.hip's BWD_LOAD_TILES has the reasons).
+constexpr uint32_t ORDER_COUNT = 0x3fffffffu, ORDER_LONG_FLAT = 0x40000000u, ORDER_LONG_IMAGE = 0x80000000u;
+constexpr uint64_t LOAD_IMAGE = 1228, LOAD_FLAT = 1434;
+
 // Screen tiles are visited in vertical strips TILE_STRIP tiles wide (the last
 // strip takes the remainder), row by row inside a strip; 0 = row-major over
 // the whole image.  Consecutive waves then cover a compact screen region

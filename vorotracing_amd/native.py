@@ -112,6 +112,12 @@ def num_tiles(images: int, H: int, W: int, tile_h: int = IMAGE_MIN, tile_w: int 
     return int(images) * ((int(H) + tile_h - 1) // tile_h) * ((int(W) + tile_w - 1) // tile_w)
 
 
+# vt_tile_order's VT_TILE_ORDER_LOAD: the order also says how even the costs are, by which the backward takes one or four
+# lanes per ray where the number of tiles does not decide (between these; other orders end with the plain split count)
+TILE_ORDER_LOAD = 1 << 31
+LOAD_TILES = (1536, 3072)
+
+
 class TileSchedule:
     """Launch order of the screen tiles of a frame rendered again (the same
     rays or cameras on one stream; vt_tile_order): each launch records its
@@ -174,7 +180,8 @@ class TileSchedule:
         if frame is None or frame != self.frame:
             return None
         self.sorted = None
-        return self._sort(stream, self.split_waves)
+        load = TILE_ORDER_LOAD if self.split_waves and LOAD_TILES[0] < self.tiles <= LOAD_TILES[1] else 0
+        return self._sort(stream, self.split_waves | load)
 
 
 def frame_key(t: torch.Tensor):
