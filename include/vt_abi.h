@@ -196,6 +196,11 @@ int vt_trace_infer_f16(const float *points, const uint16_t *diffuse, const uint1
  * adjacency / adj_diff (same results; offsets still serve stats).  quads:
  * NULL, or the footprint tables of the two maps (vt_quad_maps; extension),
  * which the kernel then reads in place of the maps' texels (same results).
+ * Small launches without stats run four lanes per ray over the scene's own
+ * arrays and maps whatever walk and quads are (same results): at most 576
+ * tiles of 64 rays, and at most 1,792 on the default stream or, in the tiled
+ * and camera entries, without walk (for a launch that has the GPU to itself or
+ * shares it with few).
  */
 int vt_trace_infer_f16_tiled(const float *points, const uint16_t *diffuse, const uint16_t *specular,
                              uint32_t diff_res, uint32_t spec_res, const float *density, const uint32_t *adjacency,

@@ -600,13 +600,23 @@ static int launch_one(const InferArgs &a, hipStream_t stream, uint32_t slots)
 // with one wave per tile over the packed layout / with four over the scene's
 // arrays, us: 625 tiles 642 / 325, 1,024 tiles 642 / 373, 2,025 tiles 645 /
 // 627, 4,096 tiles 702 / 1,077.
-constexpr uint32_t INFER_GROUP_TILES = 1792;
+// That is for a launch alone.  On a chip that other launches fill, four lanes
+// cost more instructions for nothing: renders on 2, 3 and 4 streams at once,
+// time of four over one, 300,000 and 1M sites: 576 tiles 0.53, 0.67, 0.85;
+// 1,024 tiles 0.79, 1.12, 1.37; 1,600 tiles 1.16, 1.59, 1.91, so the tiles in
+// flight may be some 2,350.  Launches on the default stream run one after
+// another; of other streams HIP's 4 hardware queues run 4 at once, and each
+// gets a quarter of that.  Without a walk layout a tiled launch takes four lanes
+// up to the first line on any stream (one wave per tile would walk the same
+// arrays): a caller that knows what else runs chooses so.
+constexpr uint32_t INFER_GROUP_TILES = 1792, INFER_GROUP_TILES_STREAM = 576;
 
 template <int RD, int RS, bool Q8>
 static int launch_infer_rs(const InferArgs &a, bool stats, int map, hipStream_t stream, uint32_t lanes)
 {
     const uint32_t tiles = (lanes + 63) / 64;
-    if (!stats && tiles <= INFER_GROUP_TILES) {
+    const bool alone = !stream || (map != MAP_LINEAR && !a.wl_chunks);
+    if (!stats && tiles <= (alone ? INFER_GROUP_TILES : INFER_GROUP_TILES_STREAM)) {
         infer_group_kernel<RD, RS, Q8><<<tiles, GROUP_BLOCK, 0, stream>>>(a, map);
         VT_LAUNCH_CHECK("infer_group_kernel");
         return VT_OK;

@@ -294,7 +294,7 @@ class VoroTracingInfer:
         outs = []
         for k, rays in enumerate(frames):
             with torch.cuda.stream(streams[k % len(streams)]):
-                out = self.render(rays, **render_kw)
+                out = self._render(rays, in_flight=len(streams), **render_kw)
             out.record_stream(cur)  # allocated on the side stream, used on the caller's
             outs.append(out)
         for s in streams:
@@ -325,6 +325,13 @@ class VoroTracingInfer:
     def render(self, rays, start_point=None, weight_threshold=0.001, max_intersections=1024,
                cell_skip_threshold=0.0, use_warp_perm: bool = True, stats: Optional[torch.Tensor] = None):
         """vorotracing.py:627-683.  Returns f16 [..., 4]."""
+        return self._render(rays, start_point, weight_threshold, max_intersections, cell_skip_threshold, use_warp_perm,
+                            stats)
+
+    def _render(self, rays, start_point=None, weight_threshold=0.001, max_intersections=1024,
+                cell_skip_threshold=0.0, use_warp_perm: bool = True, stats: Optional[torch.Tensor] = None,
+                in_flight: Optional[int] = None):
+        """``render``, one of ``in_flight`` at once where the caller knows (native.small_render)."""
         image = use_warp_perm and rays.shape[-1] == 6 and native.screen_layout(rays.shape[:-1]) is not None
         start_point, rays_per_start = self._render_start(rays, start_point, image)
         if self.quantize == "q8":
@@ -335,7 +342,7 @@ class VoroTracingInfer:
                     self.diff_offset, self.spec_scale, self.spec_offset, weight_threshold, max_intersections,
                     cell_skip_threshold)
             return self._render_q8_native(rays, start_point, weight_threshold, max_intersections,
-                                          cell_skip_threshold, image, stats, rays_per_start)
+                                          cell_skip_threshold, image, stats, rays_per_start, in_flight)
         if not image and stats is None:
             empty = torch.empty(0, dtype=torch.int32, device=self.device)
             return ops.trace_octmap_infer(self.primal_points, self.diffuse_fp16, self.specular_fp16, self.density,
@@ -350,7 +357,8 @@ class VoroTracingInfer:
                                 cell_skip_threshold=cell_skip_threshold, stats=stats,
                                 tiled=self.TILE if image else None,
                                 schedule=self._schedule(*native.image_dims(rays)) if image else None,
-                                walk=self.walk_layout() if image else None, rays_per_start=rays_per_start,
+                                walk=self._walk_for(rays, stats, in_flight) if image else None,
+                                rays_per_start=rays_per_start,
                                 quads=self.quad_tables() if image else None)
 
     def camera_start_points(self, cameras, camera_buffer=None):
@@ -414,7 +422,14 @@ class VoroTracingInfer:
                       native._quads_ptr(self.quad_tables()), sp)
         return out
 
-    def _render_q8_native(self, rays, start_point, thr, max_int, skip, image, stats, rays_per_start=0):
+    def _walk_for(self, rays, stats, in_flight):
+        """The walk layout that a render of image-shaped rays is given."""
+        if stats is None and native.small_render(native.num_tiles(*native.image_dims(rays), *self.TILE), in_flight):
+            return None
+        return self.walk_layout()
+
+    def _render_q8_native(self, rays, start_point, thr, max_int, skip, image, stats, rays_per_start=0,
+                          in_flight=None):
         import ctypes as C
 
         rays = rays.contiguous()
@@ -440,7 +455,8 @@ class VoroTracingInfer:
                       self.primal_points.shape[0], self.adjacent_diff.data_ptr(), rays.data_ptr(), B, H, W,
                       self.TILE[0], self.TILE[1], start_point.data_ptr(), int(rays_per_start), float(thr),
                       int(max_int), float(skip), out.data_ptr(), order, cost, native._p(stats),
-                      native._walk_ptr(self.walk_layout()), native._quads_ptr(self.quad_tables()), sp)
+                      native._walk_ptr(self._walk_for(rays, stats, in_flight)),
+                      native._quads_ptr(self.quad_tables()), sp)
         else:
             _lib.call("vt_trace_infer_q8", self.primal_points.data_ptr(), self.diffuse_q8.data_ptr(),
                       self.specular_q8.data_ptr(), rd, rs, *keep, self.density.data_ptr(),

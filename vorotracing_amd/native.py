@@ -112,6 +112,19 @@ def num_tiles(images: int, H: int, W: int, tile_h: int = IMAGE_MIN, tile_w: int 
     return int(images) * ((int(H) + tile_h - 1) // tile_h) * ((int(W) + tile_w - 1) // tile_w)
 
 
+# Tiles up to which the inference kernels take four lanes per ray although other launches may be running, and alone
+# (vt_infer.hip INFER_GROUP_TILES_STREAM, INFER_GROUP_TILES)
+SMALL_RENDER_TILES, SMALL_RENDER_TILES_ALONE = 576, 1792
+
+
+def small_render(tiles: int, in_flight: Optional[int]) -> bool:
+    """Whether a render of ``tiles`` screen tiles, one of ``in_flight`` at once
+    (None: not known), is given no walk layout, so that it takes four lanes
+    per ray: up to 2,304 tiles in flight these do not get in each other's way."""
+    return in_flight is not None and SMALL_RENDER_TILES < tiles <= min(SMALL_RENDER_TILES_ALONE,
+                                                                       4 * SMALL_RENDER_TILES // in_flight)
+
+
 # vt_tile_order's VT_TILE_ORDER_LOAD: the order also says how even the costs are, by which the backward takes one or four
 # lanes per ray where the number of tiles does not decide (between these; other orders end with the plain split count)
 TILE_ORDER_LOAD = 1 << 31
