@@ -130,7 +130,7 @@ __device__ __forceinline__ uint32_t level_count(const VorTree &t, int level)
 
 enum { VOR_OK = 0, VOR_FULL = 1, VOR_DEGENERATE = 2 };
 // which table overflowed (bits of the fails[F_REASON] word)
-enum { FULL_PLANES = 1, FULL_EDGES = 2, FULL_VERTICES = 4, FULL_LISTS = 8 };
+enum { FULL_PLANES = 1, FULL_VERTICES = 4, FULL_LISTS = 8 };
 
 // Passes after the first, and their queues
 constexpr int RETRIES = 2;
@@ -1452,8 +1452,8 @@ extern "C" int vt_voronoi_build_warm(const float *points, uint32_t num_points, c
     VT_HIP_CHECK(hipStreamSynchronize(s));
     if (tail[1 + F_FULL] || tail[1 + F_DEGENERATE]) {
         set_error("Voronoi build failed for %u cells over capacity (%d planes, %d vertices, %u lists longer than %d) "
-                  "and %u degenerate cuts; first failing site %u; full tables (1 planes, 2 edges, 4 vertices, "
-                  "8 lists): %u",
+                  "and %u degenerate cuts; first failing site %u; full tables (1 planes, 4 vertices, 8 "
+                  "lists): %u",
                   tail[1 + F_FULL], VorLds<NV_LARGE>::T, VorLds<NV_LARGE>::T, big_cap_for(n), LIST_K,
                   tail[1 + F_DEGENERATE], tail[1 + F_FIRST_BAD], tail[1 + F_REASON]);
         return VT_ERR_INVALID;
