@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from vorotracing_amd import _C, ops
+from vorotracing_amd import _C, build, ops
 
 from tests import helpers as H
 
@@ -165,3 +165,14 @@ def test_quad_maps_reject_mismatched_maps():
     from vorotracing_amd import native
     with pytest.raises(ValueError, match="rows"):
         native.QuadMaps.build(torch.zeros((10, 64), dtype=torch.float16), torch.zeros((9, 64), dtype=torch.float16))
+
+
+@pytest.mark.parametrize("name,spills,found", [("_ZN2vt16bwd_group_kernelIfLi4ELi4EfEEvNS_7BwdArgsE", 3, True),
+                                               ("_ZN2vt16bwd_group_kernelIfLi4ELi4EfEEvNS_7BwdArgsE", 0, False),
+                                               ("_ZN2vt10bwd_kernelIfLi4ELi4ELb0EfEEvNS_7BwdArgsE", 3, False)])
+def test_build_refuses_spilling_four_lane_kernels(name, spills, found):
+    where = "x.hip:7:1: remark: "
+    remarks = "".join(f"{where}{line} [-Rpass-analysis=kernel-resource-usage]\n" for line in (
+        "Function Name: _ZN2vt16fwd_group_kernelIfEEvv", "    VGPRs: 107", "    VGPRs Spill: 0",
+        f"Function Name: {name}", "    VGPRs: 160", "    SGPRs Spill: 2", f"    VGPRs Spill: {spills}"))
+    assert build.spilling(remarks) == ([name] if found else [])
