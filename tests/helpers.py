@@ -252,6 +252,20 @@ def assert_one_rounding(got, sums, abs_sum, count, name=""):
     assert not g[none].any(), f"{name}: a value where nothing was added"
 
 
+def assert_launches_sum(parts, whole, half, name=""):
+    """Gradients of several launches add up to those of one launch of all their
+    rays: f32 sums in two orders, within 1e-5 of the norm, and for ``half``
+    gradients, summed in f32, one rounding a launch (2^-11 of each element, or
+    2^-25 where that is subnormal)."""
+    want, got = whole.double(), [p.double() for p in parts]
+    allow = 1e-5 * float(want.norm())
+    if half:
+        allow += 2.0 ** -11 * float(want.norm() + sum(g.norm() for g in got))
+        allow += 2.0 ** -25 * want.numel() ** 0.5 * (1 + len(got))
+    diff = float((sum(got) - want).norm())
+    assert float(want.norm()) > 0 and diff <= allow, f"{name}: {diff} > {allow}"
+
+
 def f16_train_sums(s, rays, start, thr, fw16, g16, contribution=False, **bwd_kw):
     """Absolute sums and add counts (oracle sum modes) of the f16-storage
     training call whose forward outputs are ``fw16`` and upstream gradient

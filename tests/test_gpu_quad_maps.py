@@ -2,7 +2,9 @@
 the tables against a numpy construction through the oracle's octahedral wrap,
 and renders that read them, which must equal the renders that read the maps'
 texels bit for bit (buffer, camera and drop-in renders, 4x4 and 8x8 maps) and
-stay within the oracle's bound."""
+stay within the oracle's bound.  At these sizes renders without statistics run
+four lanes per ray and read the maps either way; test_gpu_one_lane.py has the
+larger ones, which read the tables."""
 import numpy as np
 import pytest
 import torch

@@ -5,10 +5,11 @@ depth_idx, distortion, W/S totals, t_far); atomically accumulated outputs
 (contribution, all gradients) are compared with the north star's 1e-3
 relative tolerance, per element (helpers.assert_grad_close: within 1e-3 of
 the element plus 1e-6 of the tensor's largest magnitude; the GPU adds in a
-different order than the serial-per-ray CPU loop).  Outputs accumulated in
-half precision (f16 attribute storage) are held per element to the
-half-precision accumulation bound of their absolute sum and add count
-(helpers.f16_sum_bound).  The "hf8" case has the reference's 8x8 diffuse and
+different order than the serial-per-ray CPU loop).  Half outputs (f16
+attribute storage) are held per element to the half-precision accumulation
+bound of their absolute sum and add count (helpers.f16_sum_bound), as the
+oracle adds halves; test_gpu_half_sums.py holds the texture gradients to one
+rounding of their f32 sums.  The "hf8" case has the reference's 8x8 diffuse and
 8x8 specular maps.
 """
 import types
@@ -137,11 +138,11 @@ def test_bwd_parity(gpu, which, f16, extras, gscale):
         if extras:
             H.assert_grad_close(perr.cpu().numpy(), want["point_error"], "point_error")
     else:
-        # f16 storage (as in the reference): texture gradients and point_error
-        # are summed with half-precision atomics, one rounding per add, in
-        # another order than the oracle's: per element within the
-        # half-precision accumulation bound of the element's absolute sum and
-        # add count.  Points and density stay f32 atomics.
+        # f16 storage: the oracle adds halves, one rounding per add (as the
+        # reference); here point_error is added so in another order, and the
+        # texture gradients are f32 sums, rounded once.  Per element within
+        # the half-precision accumulation bound of the element's absolute sum
+        # and add count.  Points and density stay f32 atomics.
         A, K = H.f16_train_sums(s, rays, start, thr, fw, g, depth_quantiles=q, depth_idx=fw["depth_idx"],
                                 depth_grad=dg, ray_error=rerr, contribution_alpha_grad=cag, distortion_grad=distg)
         H.assert_grad_close(pg.cpu().numpy(), want["points_grad"], "points_grad", abs_sum=A["points_grad"])

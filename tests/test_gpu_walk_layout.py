@@ -1,7 +1,9 @@
 """The packed walk layout (vt_walk_layout, native.WalkLayout): its arrays
 against a numpy construction, its limits, and renders through it, which must
 be the renders of the reference's arrays bit for bit (walk statistics,
-alpha and RGB), and within the oracle's bounds."""
+alpha and RGB), and within the oracle's bounds.  At these sizes renders
+without statistics run four lanes per ray over the reference's arrays either
+way; test_gpu_one_lane.py has the larger ones, which walk the layout."""
 import numpy as np
 import pytest
 import torch
@@ -99,7 +101,8 @@ def test_packed_walk_parity(gpu, scene):
             H.assert_stats_equal(H.stats_np(st), wst)
             H.assert_infer_rgba(got, want)
             outs.append(got)
-            # without statistics (the kernel the renders run)
+            # without statistics (the kernel that renders of this size run: four lanes per ray, whatever walk is;
+            # test_gpu_one_lane.py has the larger ones, which walk the layout)
             outs.append(native.infer_f16(d["points"], d["diffuse4"], d["specular4"], d["density"], d["adjacency"],
                                          d["offsets"], d["adj"], H.to_dev(rays, gpu), H.to_dev(start, gpu),
                                          weight_threshold=0.01, cell_skip_threshold=1e-3, tiled=(8, 8), walk=walk))
