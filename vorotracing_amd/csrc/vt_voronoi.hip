@@ -35,12 +35,14 @@
 // caller's guesses), which usually leaves it near its final shape, and then
 // offered what the tree still holds within its reach.
 //
-// What bounds it: instruction issue.  The first pass runs 10,000 VALU and
-// 5,400 scalar instructions per cell (22 cuts of about 200, 33 box tests of
-// 80, 11 batches of sites of 150), the VALU busy 92 % of the time at 4 waves
-// per SIMD; the later passes are bound by their longest cells.  1M heightfield
-// sites: 144 ms with the cell in LDS and a uniform grid, 33 ms so; 262k torus
-// sites after a move, from their old adjacency: 44 and 6.3 ms.
+// What bounds it: instruction issue.  The first pass runs 9,900 VALU and 5,400
+// scalar instructions per cell (22 cuts of about 200, 33 box tests of 80, 11
+// batches of sites of 150), 10.4 G VALU instructions in 20.6 ms at 5 waves per
+// SIMD: one in flight in 90 % of the SIMDs' quad-cycles (SQ_ACTIVE_INST_VALU),
+// though an f32 one alone takes half of a quad-cycle (41 % of that peak).  The
+// later passes are bound by their longest cells.  1M heightfield sites: 131 ms
+// with the cell in LDS and a uniform grid, 33 ms so; 262k torus sites after a
+// move, from their old adjacency: 38.9 and 6.5 ms.
 #include "vt_internal.h"
 #include "vt_prims.h"
 
