@@ -967,7 +967,7 @@ def train_rooflines(model, rays, sp, g, dev, log, R=10):
 
 def train_f16_storage(model, rays, sp, g, dev, log, R=10):
     """The C2 forward and backward entries with f16 attribute storage (the reference's half-precision maps:
-    f16 textures, RGBA and its gradient; texture gradients summed with half-precision atomics), HIP events
+    f16 textures, RGBA and its gradient; texture gradients summed in f32 and rounded once), HIP events
     around R calls of each _C entry, prefetch included."""
     import torch
 

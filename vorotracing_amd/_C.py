@@ -594,8 +594,8 @@ def _stats_ptr(stats: Optional[torch.Tensor], num_rays: int):
 # texel values, or this many a ray: clearing the sums, 4 bytes a value, costs
 # less there than f32 atomics save against half ones.  Backward of 8x8 maps with
 # half atomics / with sums, ms: 3M sites (1.15e9 values) 1,024 rays 6.5 / 3.4,
-# 262,144 rays 9.0 / 8.8; 8M sites (3.1e9) 65,536 rays 9.2 / 9.3 and with ray_error 9.3 / 11.6, 262,144 rays
-# 16.5 / 17.6, a million rays 40.0 / 37.9.
+# 262,144 rays 9.0 / 8.8; 8M sites (3.1e9) 65,536 rays 9.2 / 9.3 and with
+# ray_error 9.3 / 11.6, 262,144 rays 16.5 / 17.6, a million rays 40.0 / 37.9.
 SUMS_VALUES = 1_200_000_000
 SUMS_VALUES_PER_RAY = 4096
 
