@@ -183,6 +183,20 @@ def test_coplanar_sites_on_a_tilted_plane(gpu, n):
     _check(np.concatenate([pts, up]).astype(np.float32), gpu)
 
 
+@pytest.mark.parametrize("n,sparse,depth,seed", [(10000, 20, 1e-2, 3), (3000, 30, 1e-2, 3), (10000, 10, 1e-3, 1),
+                                                 (10000, 25, 1e-3, 1)])
+def test_sparse_sites_about_a_dense_shell(gpu, n, sparse, depth, seed):
+    """Cells that see more of a dense surface, before their other neighbours
+    close them, than 512 vertices hold, and end with at most 255 neighbours."""
+    rng = np.random.default_rng(seed)
+    p = rng.normal(size=(n, 3))
+    p *= (1 - depth * rng.uniform(0, 1, (n, 1))) / np.linalg.norm(p, axis=1, keepdims=True)
+    m = n // sparse
+    up = rng.normal(size=(m, 3))
+    up *= (1.02 + rng.exponential(1.0, (m, 1))) / np.linalg.norm(up, axis=1, keepdims=True)
+    _check(np.concatenate([p, up]).astype(np.float32), gpu)
+
+
 @pytest.mark.parametrize("scale", [1e-6, 1.0, 1e6])
 def test_clusters_of_very_different_density(gpu, scale):
     """Clusters a thousandth of the scene wide beside sparse sites (a Morton

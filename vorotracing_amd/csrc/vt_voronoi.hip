@@ -25,7 +25,7 @@
 // vertex finds the boundary edges among its own three by testing bits of the
 // removed set, the new triangles go to free lanes and meet along the boundary
 // through two per-plane tables.  First pass: 64 vertices per cell (one per
-// lane); cells with more run again with 128, and then with 512.
+// lane); cells with more run again with 128, then with 512 and 1,024.
 //
 // Sites are sorted along a Morton curve and kept in a tree of bounding boxes
 // that is 64 children wide, one child per lane: 8 sites per box at the bottom.
@@ -58,13 +58,16 @@ constexpr int VOR_BLOCK = 64; // one wave
 // Neighbour lists: LIST_K entries per site; longer lists in slots of BIG_K.
 constexpr int LIST_K = 64;
 constexpr int BIG_K = 255;
-// Vertices per lane of the three passes, each of which takes the cells that
-// overflow the one before (plane slots: 64 per vertex slot; a cell of T
-// vertices has T / 2 + 2 faces, so the slots never run out first).  1M
-// heightfield sites queue 10,423 cells for the second pass and 938 for the
-// third.  A pass ends with its longest cell, 3 to 4 ms there whatever the
-// vertices per lane: a pass of 4 between the last two cost 3 ms more in all.
-constexpr int NV_SMALL = 1, NV_MID = 2, NV_LARGE = 8;
+// Vertices per lane of the passes, each of which takes the cells that overflow
+// the one before (plane slots: 64 per vertex slot; a cell of T vertices has T /
+// 2 + 2 faces, so the slots never run out first).  1M heightfield sites queue
+// 10,423 cells for the second pass and 938 for the third.  A pass ends with its
+// longest cell, 3 to 4 ms there whatever the vertices per lane: a pass of 4
+// between the second and the third cost 3 ms more in all.  The fourth runs only
+// when the host finds cells queued for it: those beside a far denser surface,
+// of which a cell sees more, before its other neighbours close it, than it
+// keeps (255 neighbours at most): one of 10,500 sites in and about a thin shell.
+constexpr int NV_SMALL = 1, NV_MID = 2, NV_LARGE = 8, NV_HUGE = 16;
 
 // The site tree: level 0 has boxes of VOR_LEAF consecutive sorted sites,
 // level k + 1 boxes of 64 boxes of level k; the walk starts at level `top`,
@@ -135,8 +138,8 @@ enum { VOR_OK = 0, VOR_FULL = 1, VOR_DEGENERATE = 2 };
 enum { FULL_PLANES = 1, FULL_VERTICES = 4, FULL_LISTS = 8 };
 
 // Passes after the first, and their queues
-constexpr int RETRIES = 2;
-template <int NV> constexpr int QUEUE_OF = NV == NV_MID ? 0 : 1;
+constexpr int RETRIES = 3;
+template <int NV> constexpr int QUEUE_OF = NV == NV_MID ? 0 : NV == NV_LARGE ? 1 : 2;
 
 // fails[] words: failures, the cells queued for each further pass and those
 // passes' work counters, big-list slots
@@ -489,10 +492,10 @@ __device__ __forceinline__ int close_hole(VorLds<NV> &s, VorCell<NV> &c, const u
             const uint64_t m = __ballot(b);
             const uint32_t at = cnt + rank_in(m);
             if (b && at < T) {
-                // edge: u | v << 10 | kept << 20 | the kept triangle's link back << 29
+                // edge: u | v << 10 | kept << 20 | the kept triangle's link back << 30
                 const ushort4 back = s.nb[to[e]];
                 const uint32_t link = back.x == me ? 0u : back.y == me ? 1u : 2u;
-                s.edge[at] = id[e] | id[(e + 1) % 3] << 10 | to[e] << 20 | link << 29;
+                s.edge[at] = id[e] | id[(e + 1) % 3] << 10 | to[e] << 20 | link << 30;
             }
             cnt += (uint32_t)__popcll(m);
         }
@@ -519,11 +522,11 @@ __device__ __forceinline__ int close_hole(VorLds<NV> &s, VorCell<NV> &c, const u
         base += (uint32_t)__popcll(f);
         fresh[k] = __ballot(mine);
         if (mine) {
-            const uint32_t me = 64u * k + (uint32_t)lane, e = s.edge[j], kept = (e >> 20) & 511u;
+            const uint32_t me = 64u * k + (uint32_t)lane, e = s.edge[j], kept = (e >> 20) & 1023u;
             edge[k] = e;
             s.by_u[e & 1023u] = c.gen << 10 | me;
             s.by_v[(e >> 10) & 1023u] = c.gen << 10 | me;
-            reinterpret_cast<uint16_t *>(&s.nb[kept])[e >> 29] = (uint16_t)me;
+            reinterpret_cast<uint16_t *>(&s.nb[kept])[e >> 30] = (uint16_t)me;
         }
     }
     lds_sync();
@@ -534,7 +537,7 @@ __device__ __forceinline__ int close_hole(VorLds<NV> &s, VorCell<NV> &c, const u
             const uint32_t me = 64u * k + (uint32_t)lane, e = edge[k];
             uint32_t next, prev;
             bad = new_vertex(s, c, k, me, e & 1023u, (e >> 10) & 1023u, pq, q, next, prev) || bad;
-            s.nb[me] = make_ushort4((uint16_t)((e >> 20) & 511u), (uint16_t)next, (uint16_t)prev, 0);
+            s.nb[me] = make_ushort4((uint16_t)((e >> 20) & 1023u), (uint16_t)next, (uint16_t)prev, 0);
         }
         c.alive[k] = (c.alive[k] & ~out[k]) | fresh[k];
     }
@@ -546,7 +549,7 @@ __device__ __forceinline__ int close_hole(VorLds<NV> &s, VorCell<NV> &c, const u
 // every lane tests its vertices, and the cell changes only when some lie
 // outside.  Sites on common spheres make vertices of one place, which rounding
 // may part to both sides of a plane through it, so that what a cut removes is
-// no disc.  The last pass, which takes such cells too, therefore leaves the
+// no disc.  The last passes, which take such cells too, therefore leave the
 // vertices within ON_PLANE |x| |v| of a plane (the rounding of x.v and of v, 500
 // times) on it; a second site at the place of a neighbour still fails.
 constexpr double ON_PLANE = 1e-13;
@@ -565,7 +568,7 @@ __device__ __forceinline__ int cell_cut(VorLds<NV> &s, VorCell<NV> &c, const Vor
             continue;
         const double xv = fma(dx, c.v[k].x, fma(dy, c.v[k].y, dz * c.v[k].z));
         const bool o = xv > w;
-        if (NV == NV_LARGE) {
+        if (NV >= NV_LARGE) {
             // (above) only what is outside by more than rounding is removed
             any |= __ballot(o) & c.alive[k];
             out[k] = __ballot(xv - w > ON_PLANE * sqrt(2.0 * w) * (double)c.fl[k]) & c.alive[k];
@@ -582,7 +585,7 @@ __device__ __forceinline__ int cell_cut(VorLds<NV> &s, VorCell<NV> &c, const Vor
     }
     if (!any)
         return VOR_OK;
-    if (NV == NV_LARGE) {
+    if (NV >= NV_LARGE) {
         bool twin = false;
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
@@ -961,8 +964,8 @@ template <int NV> __device__ __forceinline__ void cell_drop_flat(VorLds<NV> &s, 
 // on one side make long slivers, whose vertices lose their digits.  The third
 // pass goes in smaller steps.  FAR_TIMES: distance, in radii of the first
 // ball, beyond which a vertex counts as far.
-template <int NV> constexpr int BALL_SITES = NV != NV_LARGE ? 16 : 6;
-template <int NV> constexpr float GROW2 = NV != NV_LARGE ? 4.0f : 2.0f;
+template <int NV> constexpr int BALL_SITES = NV < NV_LARGE ? 16 : 6;
+template <int NV> constexpr float GROW2 = NV < NV_LARGE ? 4.0f : 2.0f;
 constexpr float FAR_TIMES = 4.0f;
 
 // Voronoi cell of the site at sorted position `at`; its neighbours go to
@@ -1117,8 +1120,8 @@ __device__ __forceinline__ void cell_and_list(VorLds<NV> &s, VorCell<NV> &c, con
     } else {
         m = 0;
         if (lane == 0) {
-            if (NV != NV_LARGE && !(c.full & FULL_LISTS)) {
-                constexpr int next = NV == NV_SMALL ? QUEUE_OF<NV_MID> : QUEUE_OF<NV_LARGE>;
+            if (NV != NV_HUGE && (NV != NV_LARGE || status == VOR_FULL) && !(c.full & FULL_LISTS)) {
+                constexpr int next = NV == NV_SMALL ? QUEUE_OF<NV_MID> : NV == NV_MID ? QUEUE_OF<NV_LARGE> : QUEUE_OF<NV_HUGE>;
                 o.retry[next][atomicAdd(o.fails + F_RETRY + next, 1u)] = at; // at most n entries
             } else {
                 atomicAdd(o.fails + (status == VOR_FULL ? F_FULL : F_DEGENERATE), 1u);
@@ -1312,7 +1315,7 @@ __global__ void voronoi_begin_kernel(uint32_t *fails, uint32_t *last_count, cons
 
 // workspace layout (u32 words)
 struct VorWs {
-    uint32_t *lists, *counts, *keys, *keys_lo, *vals, *sort_ws, *scan_ws, *fails, *bbox_ws, *retry[RETRIES], *big_lists,
+    uint32_t *lists, *counts, *keys, *keys_lo, *vals, *sort_ws, *scan_ws, *fails, *bbox_ws, *retry[RETRIES - 1], *big_lists,
         *big_slot, *sites, *boxes;
     float *bbox;
     VorBox *box;
@@ -1349,8 +1352,8 @@ static size_t ws_words(uint32_t n, VorWs *w, uint32_t *base)
     x.bbox = reinterpret_cast<float *>(bb);
     take(&bb, sizeof(VorBox) / 4); // (each of these starts at a multiple of 256 bytes)
     x.box = reinterpret_cast<VorBox *>(bb);
-    for (int q = 0; q < RETRIES; ++q)
-        take(&x.retry[q], n);
+    for (uint32_t *&queue : x.retry)
+        take(&queue, n);
     take(&x.big_lists, (size_t)big_cap_for(n) * BIG_K);
     take(&x.big_slot, n);
     take(&x.sites, 4 * (size_t)n);
@@ -1430,7 +1433,8 @@ extern "C" int vt_voronoi_build_warm(const float *points, uint32_t num_points, c
         voronoi_level_kernel<<<w.count[t.top], 64, 0, s>>>(below, nbelow, boxes + 2 * (size_t)level_begin(t, t.top));
         VT_LAUNCH_CHECK("voronoi_level_kernel");
     }
-    VorLists o{w.lists, w.big_lists, w.big_slot, w.counts, big_cap_for(n), {w.retry[0], w.retry[1]}, w.fails};
+    // (the third pass queues for the fourth where the second's queue was)
+    VorLists o{w.lists, w.big_lists, w.big_slot, w.counts, big_cap_for(n), {w.retry[0], w.retry[1], w.retry[0]}, w.fails};
     const uint32_t per = std::min<uint32_t>(8, std::max<uint32_t>(1, n / 32768));
     const uint32_t blocks = (n + per - 1) / per;
     // cold builds run an instantiation without any of the warm-start code
@@ -1445,18 +1449,25 @@ extern "C" int vt_voronoi_build_warm(const float *points, uint32_t num_points, c
     VT_LAUNCH_CHECK("voronoi_retry_kernel (second pass)");
     voronoi_retry_kernel<NV_LARGE><<<std::min<uint32_t>(n, 1024), VOR_BLOCK, 0, s>>>(points, t, n, o);
     VT_LAUNCH_CHECK("voronoi_retry_kernel (third pass)");
-    rc = exclusive_scan_u32(w.counts, offsets, n + 1, w.scan_ws, s);
-    if (rc)
-        return rc;
     uint32_t tail[1 + F_WORDS];
-    VT_HIP_CHECK(hipMemcpyAsync(tail, offsets + n, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    VT_HIP_CHECK(hipMemcpyAsync(tail + 1, w.fails, F_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    VT_HIP_CHECK(hipStreamSynchronize(s));
+    for (int huge = 0; huge < 2; ++huge) {
+        rc = exclusive_scan_u32(w.counts, offsets, n + 1, w.scan_ws, s);
+        if (rc)
+            return rc;
+        VT_HIP_CHECK(hipMemcpyAsync(tail, offsets + n, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        VT_HIP_CHECK(hipMemcpyAsync(tail + 1, w.fails, F_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        VT_HIP_CHECK(hipStreamSynchronize(s));
+        const uint32_t queued = tail[1 + F_RETRY + QUEUE_OF<NV_HUGE>];
+        if (huge || !queued || tail[1 + F_FULL] || tail[1 + F_DEGENERATE])
+            break;
+        voronoi_retry_kernel<NV_HUGE><<<std::min<uint32_t>(queued, 512), VOR_BLOCK, 0, s>>>(points, t, n, o);
+        VT_LAUNCH_CHECK("voronoi_retry_kernel (fourth pass)");
+    }
     if (tail[1 + F_FULL] || tail[1 + F_DEGENERATE]) {
         set_error("Voronoi build failed for %u cells over capacity (%d planes, %d vertices, %u lists longer than %d) "
                   "and %u degenerate cuts; first failing site %u; full tables (1 planes, 4 vertices, 8 "
                   "lists): %u",
-                  tail[1 + F_FULL], VorLds<NV_LARGE>::T, VorLds<NV_LARGE>::T, big_cap_for(n), LIST_K,
+                  tail[1 + F_FULL], VorLds<NV_HUGE>::T, VorLds<NV_HUGE>::T, big_cap_for(n), LIST_K,
                   tail[1 + F_DEGENERATE], tail[1 + F_FIRST_BAD], tail[1 + F_REASON]);
         return VT_ERR_INVALID;
     }
