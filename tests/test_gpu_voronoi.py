@@ -183,6 +183,44 @@ def test_coplanar_sites_on_a_tilted_plane(gpu, n):
     _check(np.concatenate([pts, up]).astype(np.float32), gpu)
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("n", [7, 50, 200])
+def test_coplanar_sites_on_a_circle(gpu, n, axis):
+    """Sites on a circle, in f32 and so not quite: their cells are columns that
+    all meet within 1e-7 of its centre, with faces down to 1e-10 wide there.
+    Neighbours of the plane's own Delaunay triangulation."""
+    from scipy.spatial import Delaunay
+
+    a = np.random.default_rng(4).uniform(0, 2 * np.pi, n)
+    flat = np.unique(np.stack([np.cos(a), np.sin(a)], axis=1).astype(np.float32), axis=0)
+    ptr, idx = Delaunay(flat.astype(np.float64)).vertex_neighbor_vertices
+    adj, off, _ = ops.build_voronoi_adjacency(H.to_dev(np.ascontiguousarray(np.insert(flat, axis, 0.0, axis=1)), gpu))
+    adj, off = adj.cpu().numpy(), off.cpu().numpy()
+    for i in range(len(flat)):
+        assert np.array_equal(adj[off[i]:off[i + 1]], np.sort(idx[ptr[i]:ptr[i + 1]])), i
+
+
+@pytest.mark.parametrize("tilt", [False, True])
+@pytest.mark.parametrize("w,h", [(2, 2), (5, 40), (30, 31)])
+def test_coplanar_grid(gpu, w, h, tilt):
+    """A grid in a plane (tilted: of rectangles, in z = x): four sites on every
+    circle, whose diagonal columns touch in a line and are no neighbours, in a
+    cold build and from guesses that hold them."""
+    i, j = (x.ravel() for x in np.meshgrid(np.arange(w), np.arange(h), indexing="ij"))
+    pts = np.stack([i, j, i if tilt else 0 * i], axis=1).astype(np.float32)
+    near = np.maximum(abs(i[:, None] - i), abs(j[:, None] - j)) == 1
+    side = near & (abs(i[:, None] - i) + abs(j[:, None] - j) == 1)
+    want = [np.nonzero(x)[0] for x in side]
+    guess = [np.nonzero(x)[0] for x in near]
+    guesses = dict(initial_guesses=H.to_dev(np.concatenate(guess).astype(np.uint32), gpu),
+                   initial_guesses_offsets=H.to_dev(np.cumsum([0] + [len(g) for g in guess]).astype(np.uint32), gpu))
+    for kw in ({}, guesses):
+        adj, off, _ = ops.build_voronoi_adjacency(H.to_dev(pts, gpu), **kw)
+        adj, off = adj.cpu().numpy(), off.cpu().numpy()
+        for c in range(len(pts)):
+            assert np.array_equal(adj[off[c]:off[c + 1]], want[c]), c
+
+
 @pytest.mark.parametrize("n,sparse,depth,seed", [(10000, 20, 1e-2, 3), (3000, 30, 1e-2, 3), (10000, 10, 1e-3, 1),
                                                  (10000, 25, 1e-3, 1)])
 def test_sparse_sites_about_a_dense_shell(gpu, n, sparse, depth, seed):

@@ -899,27 +899,58 @@ __device__ __forceinline__ void cell_begin(VorLds<NV> &s, VorCell<NV> &c, const 
 // places lose their mark in s.used, so that the neighbours do not depend on the
 // order.  Only a cell with two linked vertices in one place can have any
 // (SAME_PLACE |v| apart, some dozen roundings: in general position there are none).
+//
+// At a vertex on a box plane, 10^6 extents away, that is 10^-8 of an extent, and
+// the cells of coplanar sites are columns as wide there as at the site.  Two of
+// them are in one place if the lines that end in them also meet the plane
+// through the site alongside the box plane in one, by the measure of that place
+// (by the far one alone, 7 of the 97 pairs of neighbours among 50 sites on a
+// circle, rounded to f32, were lost).
 constexpr double SAME_PLACE = 1e-14;
-__device__ __forceinline__ bool same_place(double4 a, double x, double y, double z, float len)
+__device__ __forceinline__ bool same_place(d3 a, d3 b, float len)
 {
-    return fmax(fmax(fabs(a.x - x), fabs(a.y - y)), fabs(a.z - z)) <= SAME_PLACE * (double)len;
+    return fmax(fmax(fabs(a.x - b.x), fabs(a.y - b.y)), fabs(a.z - b.z)) <= SAME_PLACE * (double)len;
+}
+__device__ __forceinline__ d3 readlane_d3(d3 x, int l)
+{
+    return d3{readlane_d(x.x, l), readlane_d(x.y, l), readlane_d(x.z, l)};
 }
 template <int NV> __device__ __forceinline__ void cell_drop_flat(VorLds<NV> &s, const VorCell<NV> &c, int lane)
 {
+    // where the line of a vertex on one box plane passes the site (other
+    // vertices: themselves), and that plane (others: 6)
+    d3 at[NV];
+    uint32_t wall[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        at[k] = c.v[k];
+        wall[k] = 6;
+        if (!c.farv[k]) // (no vertex on a box plane)
+            continue;
+        const uint32_t a = c.tri[k] & 1023u, b = (c.tri[k] >> 10) & 1023u, d = c.tri[k] >> 20;
+        const uint32_t low = min(a, min(b, d));
+        if (((c.alive[k] >> lane) & 1u) && low < 6u && max(min(a, b), min(max(a, b), d)) >= 6u) {
+            double4 w[3] = {s.P[a], s.P[b], s.P[d]};
+            (low == a ? w[0] : low == b ? w[1] : w[2]).w = 0.0;
+            at[k] = plane_vertex(w[0], w[1], w[2]);
+            wall[k] = low;
+        }
+    }
     // the planes are no longer needed: vertex positions take their place
     lds_sync();
 #pragma unroll
     for (int k = 0; k < NV; ++k)
         s.P[64 * k + lane] = make_double4(c.v[k].x, c.v[k].y, c.v[k].z, 0.0);
     lds_sync();
+    auto place_of = [&](uint32_t v) { return d3{s.P[v].x, s.P[v].y, s.P[v].z}; };
     bool close = false;
 #pragma unroll
     for (int k = 0; k < NV; ++k)
         if ((c.alive[k] >> lane) & 1u) {
             const auto n = s.nb[64 * k + lane];
-            const double x = c.v[k].x, y = c.v[k].y, z = c.v[k].z;
-            close = close || same_place(s.P[n.x], x, y, z, c.fl[k]) || same_place(s.P[n.y], x, y, z, c.fl[k]) ||
-                    same_place(s.P[n.z], x, y, z, c.fl[k]);
+            const d3 v = c.v[k];
+            close = close || same_place(place_of(n.x), v, c.fl[k]) || same_place(place_of(n.y), v, c.fl[k]) ||
+                    same_place(place_of(n.z), v, c.fl[k]);
         }
     if (!__ballot(close))
         return;
@@ -928,24 +959,38 @@ template <int NV> __device__ __forceinline__ void cell_drop_flat(VorLds<NV> &s, 
             continue;
         uint64_t on[NV];
         uint32_t first = 0, second = 0;
+        d3 first_at{0.0, 0.0, 0.0}, second_at{0.0, 0.0, 0.0};
+        uint32_t first_wall = 6, second_wall = 6;
 #pragma unroll
         for (int k = NV - 1; k >= 0; --k) {
             const uint32_t t = c.tri[k];
             on[k] = __ballot((t & 1023u) == q || ((t >> 10) & 1023u) == q || t >> 20 == q) & c.alive[k];
-            if (on[k])
-                first = 64u * k + (uint32_t)__builtin_ctzll(on[k]);
+            if (on[k]) {
+                const int l = (int)__builtin_ctzll(on[k]);
+                first = 64u * k + (uint32_t)l;
+                first_at = readlane_d3(at[k], l);
+                first_wall = (uint32_t)__builtin_amdgcn_readlane((int)wall[k], l);
+            }
         }
         bool flat = true;
         for (int place = 0; place < 2 && flat; ++place) {
             // the vertices of the face that are elsewhere
-            const double4 p = s.P[place ? second : first];
+            const d3 p = place_of(place ? second : first), p_at = place ? second_at : first_at;
+            const uint32_t p_wall = place ? second_wall : first_wall;
             uint64_t any = 0;
 #pragma unroll
             for (int k = NV - 1; k >= 0; --k) {
-                on[k] &= __ballot(!same_place(p, c.v[k].x, c.v[k].y, c.v[k].z, c.fl[k]));
+                const d3 x = at[k];
+                const float len = wall[k] == 6u ? c.fl[k] : (float)sqrt(fma(x.x, x.x, fma(x.y, x.y, x.z * x.z)));
+                const bool same = wall[k] == p_wall && same_place(p, c.v[k], c.fl[k]) && same_place(p_at, x, len);
+                on[k] &= __ballot(!same);
                 any |= on[k];
-                if (on[k])
-                    second = 64u * k + (uint32_t)__builtin_ctzll(on[k]);
+                if (on[k]) {
+                    const int l = (int)__builtin_ctzll(on[k]);
+                    second = 64u * k + (uint32_t)l;
+                    second_at = readlane_d3(x, l);
+                    second_wall = (uint32_t)__builtin_amdgcn_readlane((int)wall[k], l);
+                }
             }
             if (!any)
                 break;
