@@ -184,15 +184,18 @@ def test_coplanar_sites_on_a_tilted_plane(gpu, n):
 
 
 @pytest.mark.parametrize("axis", [0, 1, 2])
-@pytest.mark.parametrize("n", [7, 50, 200])
-def test_coplanar_sites_on_a_circle(gpu, n, axis):
+@pytest.mark.parametrize("n,hub,seed", [(7, False, 4), (50, False, 4), (200, False, 4), (240, True, 11), (240, True, 15),
+                                        (100, True, 0)])
+def test_coplanar_sites_on_a_circle(gpu, n, hub, seed, axis):
     """Sites on a circle, in f32 and so not quite: their cells are columns that
-    all meet within 1e-7 of its centre, with faces down to 1e-10 wide there.
-    Neighbours of the plane's own Delaunay triangulation."""
+    all meet within 1e-7 of its centre, with faces down to 1e-10 wide there; with
+    a site at the centre (hub), a column that some of the others cut by less
+    than 1e-7.  Neighbours of the plane's own Delaunay triangulation."""
     from scipy.spatial import Delaunay
 
-    a = np.random.default_rng(4).uniform(0, 2 * np.pi, n)
-    flat = np.unique(np.stack([np.cos(a), np.sin(a)], axis=1).astype(np.float32), axis=0)
+    a = np.random.default_rng(seed).uniform(0, 2 * np.pi, n)
+    flat = np.concatenate([np.zeros((int(hub), 2)), np.stack([np.cos(a), np.sin(a)], axis=1)]).astype(np.float32)
+    flat = np.unique(flat, axis=0)
     ptr, idx = Delaunay(flat.astype(np.float64)).vertex_neighbor_vertices
     adj, off, _ = ops.build_voronoi_adjacency(H.to_dev(np.ascontiguousarray(np.insert(flat, axis, 0.0, axis=1)), gpu))
     adj, off = adj.cpu().numpy(), off.cpu().numpy()

@@ -545,13 +545,31 @@ __device__ __forceinline__ int close_hole(VorLds<NV> &s, VorCell<NV> &c, const u
     return __ballot(bad) ? VOR_DEGENERATE : VOR_OK;
 }
 
+// The box plane of a vertex that lies on one of them (else 6), and where the
+// line that ends there meets the plane through the site alongside it.  A vertex
+// 10^6 extents away has 6 digits fewer than that place, and the cells of
+// coplanar sites are columns as wide there as at the site.
+template <int NV> __device__ __forceinline__ uint32_t wall_of(const VorLds<NV> &s, uint32_t tri, d3 &at)
+{
+    const uint32_t a = tri & 1023u, b = (tri >> 10) & 1023u, d = tri >> 20, low = min(a, min(b, d));
+    if (low >= 6u || max(min(a, b), min(max(a, b), d)) < 6u)
+        return 6;
+    double4 w[3] = {s.P[a], s.P[b], s.P[d]};
+    (low == a ? w[0] : low == b ? w[1] : w[2]).w = 0.0;
+    at = plane_vertex(w[0], w[1], w[2]);
+    return low;
+}
+
 // Cut by the bisector of `site` at q (wave-uniform; the cell's own site at p):
 // every lane tests its vertices, and the cell changes only when some lie
 // outside.  Sites on common spheres make vertices of one place, which rounding
 // may part to both sides of a plane through it, so that what a cut removes is
 // no disc.  The last passes, which take such cells too, therefore leave the
 // vertices within ON_PLANE |x| |v| of a plane (the rounding of x.v and of v, 500
-// times) on it; a second site at the place of a neighbour still fails.
+// times) on it; a second site at the place of a neighbour still fails.  For a
+// vertex on a box plane that is 10^-7 of an extent, the depth to which one of
+// 240 coplanar sites on a circle cuts the cell of a site within: where it is so
+// near the plane, its line decides at the site.
 constexpr double ON_PLANE = 1e-13;
 template <int NV, bool WARM>
 __device__ __forceinline__ int cell_cut(VorLds<NV> &s, VorCell<NV> &c, const VorReach &p, float qx, float qy, float qz,
@@ -560,7 +578,7 @@ __device__ __forceinline__ int cell_cut(VorLds<NV> &s, VorCell<NV> &c, const Vor
     const double dx = (double)qx - (double)p.px, dy = (double)qy - (double)p.py, dz = (double)qz - (double)p.pz;
     const double w = 0.5 * fma(dx, dx, fma(dy, dy, dz * dz));
     uint64_t out[NV];
-    uint64_t any = 0, kept = 0, clear = 0;
+    uint64_t any = 0, kept = 0, clear = 0, on_plane = 0;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         out[k] = 0;
@@ -570,8 +588,10 @@ __device__ __forceinline__ int cell_cut(VorLds<NV> &s, VorCell<NV> &c, const Vor
         const bool o = xv > w;
         if (NV >= NV_LARGE) {
             // (above) only what is outside by more than rounding is removed
-            any |= __ballot(o) & c.alive[k];
+            const uint64_t cut = __ballot(o) & c.alive[k];
+            any |= cut;
             out[k] = __ballot(xv - w > ON_PLANE * sqrt(2.0 * w) * (double)c.fl[k]) & c.alive[k];
+            on_plane |= cut & ~out[k];
             s.gone[64 * k + lane] = (out[k] >> lane) & 1u;
             kept |= c.alive[k] & ~out[k];
             clear |= out[k];
@@ -586,6 +606,22 @@ __device__ __forceinline__ int cell_cut(VorLds<NV> &s, VorCell<NV> &c, const Vor
     if (!any)
         return VOR_OK;
     if (NV >= NV_LARGE) {
+        if (on_plane) {
+            kept = 0;
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                if (!c.alive[k])
+                    continue;
+                bool o = ((c.alive[k] & ~out[k]) >> lane & 1u) && fma(dx, c.v[k].x, fma(dy, c.v[k].y, dz * c.v[k].z)) > w;
+                d3 at;
+                o = o && wall_of(s, c.tri[k], at) < 6u &&
+                    fma(dx, at.x, fma(dy, at.y, dz * at.z)) - w > ON_PLANE * sqrt(2.0 * w * dot_d(at, at));
+                out[k] |= __ballot(o);
+                s.gone[64 * k + lane] = (out[k] >> lane) & 1u;
+                kept |= c.alive[k] & ~out[k];
+                clear |= out[k];
+            }
+        }
         bool twin = false;
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
@@ -900,12 +936,10 @@ __device__ __forceinline__ void cell_begin(VorLds<NV> &s, VorCell<NV> &c, const 
 // order.  Only a cell with two linked vertices in one place can have any
 // (SAME_PLACE |v| apart, some dozen roundings: in general position there are none).
 //
-// At a vertex on a box plane, 10^6 extents away, that is 10^-8 of an extent, and
-// the cells of coplanar sites are columns as wide there as at the site.  Two of
-// them are in one place if the lines that end in them also meet the plane
-// through the site alongside the box plane in one, by the measure of that place
-// (by the far one alone, 7 of the 97 pairs of neighbours among 50 sites on a
-// circle, rounded to f32, were lost).
+// At a vertex on a box plane that is 10^-8 of an extent.  Two of them are in one
+// place if their lines also pass the site in one (wall_of), by the measure of
+// that place (by the far one alone, 7 of the 97 pairs of neighbours among 50
+// sites on a circle, rounded to f32, were lost).
 constexpr double SAME_PLACE = 1e-14;
 __device__ __forceinline__ bool same_place(d3 a, d3 b, float len)
 {
@@ -917,8 +951,7 @@ __device__ __forceinline__ d3 readlane_d3(d3 x, int l)
 }
 template <int NV> __device__ __forceinline__ void cell_drop_flat(VorLds<NV> &s, const VorCell<NV> &c, int lane)
 {
-    // where the line of a vertex on one box plane passes the site (other
-    // vertices: themselves), and that plane (others: 6)
+    // wall_of every vertex (at: itself where there is none)
     d3 at[NV];
     uint32_t wall[NV];
 #pragma unroll
@@ -927,14 +960,8 @@ template <int NV> __device__ __forceinline__ void cell_drop_flat(VorLds<NV> &s, 
         wall[k] = 6;
         if (!c.farv[k]) // (no vertex on a box plane)
             continue;
-        const uint32_t a = c.tri[k] & 1023u, b = (c.tri[k] >> 10) & 1023u, d = c.tri[k] >> 20;
-        const uint32_t low = min(a, min(b, d));
-        if (((c.alive[k] >> lane) & 1u) && low < 6u && max(min(a, b), min(max(a, b), d)) >= 6u) {
-            double4 w[3] = {s.P[a], s.P[b], s.P[d]};
-            (low == a ? w[0] : low == b ? w[1] : w[2]).w = 0.0;
-            at[k] = plane_vertex(w[0], w[1], w[2]);
-            wall[k] = low;
-        }
+        if ((c.alive[k] >> lane) & 1u)
+            wall[k] = wall_of(s, c.tri[k], at[k]);
     }
     // the planes are no longer needed: vertex positions take their place
     lds_sync();
