@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from tests import helpers as H
-from vorotracing_amd import _C, _lib, camera, scene
+from vorotracing_amd import _C, _lib, camera, native, scene
 from vorotracing_amd.infer import VoroTracingInfer
 from vorotracing_amd.model import VoroTracing
 
@@ -218,3 +218,59 @@ def test_backward_chosen_by_the_load(gpu, even, flat):
     assert long == (not even) and bool(word & (1 << (30 if flat else 31))) == long
     for a, b in zip(*got):
         assert float((a.double() - b.double()).norm()) <= 1e-5 * float(a.double().norm()) and float(a.abs().sum()) > 0
+
+
+def _ragged_scene(gpu, which):
+    """Cells with lists of 0 to 300 random neighbours (around 24, the faces that
+    four lanes search at once), sites snapped so that exit distances tie, or of
+    such sizes that face records and quotients leave their range."""
+    rng = np.random.default_rng(len(which))
+    n = 600
+    nf = rng.choice([0, 1, 3, 4, 5, 23, 24, 25, 26, 47, 48, 49, 71, 300], size=n, p=[.02] + [.07] * 2 + [.08] * 10 + [.04])
+    off = np.concatenate([[0], np.cumsum(nf)]).astype(np.uint32)
+    adj = np.concatenate([rng.integers(0, n, off[-1]), np.zeros(32, np.int64)]).astype(np.uint32)
+    pts = rng.uniform(-1, 1, size=(n, 3))
+    if which == "ties":
+        pts = np.round(pts * 2) / 2
+    elif which == "large":
+        pts *= 10.0 ** rng.uniform(0, 30, size=(n, 1))
+    elif which == "small":
+        pts *= 10.0 ** rng.uniform(-40, 0, size=(n, 1))
+    elif which == "not finite":
+        pts[rng.integers(0, n, 40), rng.integers(0, 3, 40)] = rng.choice([np.nan, np.inf, -np.inf], 40)
+    rays = rng.normal(size=(40, 48, 6))
+    if which == "ties":
+        rays = np.round(rays)
+    with np.errstate(over="ignore"):
+        a = dict(points=pts.astype(np.float32), adjacency=adj, offsets=off, rays=rays.astype(np.float32),
+                 diffuse=rng.normal(size=(n, 64)).astype(np.float16), specular=rng.normal(size=(n, 64)).astype(np.float16),
+                 density=np.exp(rng.normal(-3, 1, size=n)).astype(np.float32),
+                 start=rng.integers(0, n, size=(40, 48)).astype(np.uint32))
+    return {k: H.to_dev(v, gpu) for k, v in a.items()}
+
+
+def _same_bits(a, b):
+    """Equal bit for bit, any NaN as another."""
+    if a.is_floating_point():
+        return bool(((a == b) & (torch.signbit(a) == torch.signbit(b)) | a.isnan() & b.isnan()).all())
+    return torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("which", ["plain", "ties", "large", "small", "not finite"])
+def test_ragged_lists_and_hard_quotients(gpu, which):
+    """Renders and training forwards of few tiles, four lanes per ray, against
+    the same calls with statistics, one lane per ray."""
+    s = _ragged_scene(gpu, which)
+    adj_diff = native.prefetch(s["points"], s["adjacency"], s["offsets"])
+    for shape, tiled in (((40, 48), (8, 8)), ((1920,), None)):
+        rays, start = s["rays"].reshape(*shape, 6), s["start"].reshape(shape)
+        got = [native.infer_f16(s["points"], s["diffuse"], s["specular"], s["density"], s["adjacency"], s["offsets"],
+                                adj_diff, rays, start, weight_threshold=1e-4, max_intersections=60, stats=st, tiled=tiled)
+               for st in (None, native.new_stats(1920, gpu))]
+        assert _same_bits(*got) and bool((got[0][..., 3] > 0.1).any())
+        maps = [s[k].float()[:, :48].contiguous() for k in ("diffuse", "specular")]
+        q = torch.tensor([0.7, 0.3], device=gpu).expand(*shape, 2).contiguous()
+        out = [_C.trace_vorotracing_fwd(s["points"], *maps, s["density"].reshape(-1, 1), s["adjacency"], s["offsets"], rays,
+                                        start, q, 1e-4, 60, False, stats=st) for st in (None, native.new_stats(1920, gpu))]
+        for a, b in zip(*out):
+            assert a is None and b is None or _same_bits(a, b)
